@@ -1,0 +1,104 @@
+"""GPU tests of the token-tile projections (batches and prompts of more
+vectors than the operand groups of one pass hold): they keep the sums of the
+single-vector calls, so every comparison is bit for bit.
+
+Sizes: a small layer (hidden 160: fewer k-steps than the eight classes of the
+sum; 161 row blocks: no multiple of any workgroup's), batches at the edges of
+16-vector blocks, 64-vector tiles and of both layouts' ranges."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+HID, NQK, NV = 160, 2, 8
+CH = (2 * NQK + NV) * 128
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from vx27_amd import lib as L
+    c = L.Ctx(0)
+    yield c
+    c.close()
+
+
+def weights(ctx, r, conv_bf16=True):
+    from vx27_amd import workloads as W
+    bf = lambda shape, std: W.bf16_bits(W.normal(r, shape, std))
+    cw = W.normal(r, (CH, 4), 0.2)
+    host = {"A_log": W.normal(r, NV, 0.5), "dt_bias": W.normal(r, NV, 0.1), "norm_w": 1 + W.normal(r, 128, 0.1),
+            "conv_w": W.bf16_bits(cw) if conv_bf16 else cw}
+    dev = {k: ctx.put(v) for k, v in host.items()}
+    dev["w_in"] = ctx.put_tiled(bf((CH + NV * 128 + 2 * NV, HID), 0.1))
+    dev["w_out"] = ctx.put_tiled(bf((HID, NV * 128), 0.03))
+    dev["dt"] = 1 if conv_bf16 else 0
+    return dev
+
+
+def decode(ctx, dev, x, S, conv, skew=0):
+    """One layer step of x [B][HID]; the conv state `skew` floats off its buffer's start."""
+    from vx27_amd import lib as L
+    B = x.shape[0]
+    cs = np.concatenate([np.zeros(skew, np.float32), conv.ravel()])
+    Sd, cd, xb, ob = ctx.put(S), ctx.put(cs), ctx.put(x), ctx.buf(B * HID * 4)
+    d = L.DnLayerDesc(B, NQK, NV, 128, HID, xb.ptr, None, dev["w_in"].ptr, dev["w_out"].ptr, dev["conv_w"].ptr,
+                      dev["dt"], dev["A_log"].ptr, dev["dt_bias"].ptr, dev["norm_w"].ptr, Sd.ptr, cd.ptr + 4 * skew,
+                      ob.ptr)
+    L.check(L.lib().vx27_hip_dn_layer_decode(ctx.h, C.byref(d)), "dn_layer")
+    res = (ob.download((B, HID), np.float32), Sd.download(S.shape, np.float32),
+           cd.download(cs.shape, np.float32)[skew:].reshape(conv.shape))
+    for b in (Sd, cd, xb, ob):
+        b.free()
+    return res
+
+
+def inputs(r, B):
+    from vx27_amd import workloads as W
+    return W.normal(r, (B, HID)), W.normal(r, (B, NV, 128, 128), 0.02), W.normal(r, (B, CH, 3), 0.5)
+
+
+@pytest.mark.parametrize("B,conv_bf16,skew", [(35, True, 0), (36, True, 0), (48, False, 0), (49, True, 1), (64, True, 0),
+                                              (65, False, 1), (66, True, 0), (131, True, 0)])
+def test_decode_batch_bits(ctx, B, conv_bf16, skew):
+    """A batch gives the bits of its sequences one by one (outputs, states and
+    conv states; unaligned conv states too)."""
+    from vx27_amd import workloads as W
+    r = W.rng(31, f"tok_decode_{B}")
+    dev = weights(ctx, r, conv_bf16)
+    x, S, conv = inputs(r, B)
+    got = decode(ctx, dev, x, S, conv, skew)
+    for b in sorted({0, 1, 15, 16, 33, 34, B // 2, B - 2, B - 1}):
+        one = decode(ctx, dev, x[b:b + 1], S[b:b + 1], conv[b:b + 1])
+        for g, o, n in zip(got, one, ("out", "S", "conv")):
+            assert np.array_equal(g[b], o[0]), (n, b)
+
+
+@pytest.mark.parametrize("T", [36, 66, 255])
+def test_gqa_prompt_cache_bits(ctx, T):
+    """The cache rows of a prompt in one call and in single-token calls (bf16
+    segments of the token tiles and of the operand groups)."""
+    from vx27_amd import lib as L, workloads as W
+    r = W.rng(33, f"tok_gqa_{T}")
+    bf = lambda shape, std: W.bf16_bits(W.normal(r, shape, std))
+    wq, wo = ctx.put_tiled(bf((24 * 512 + 2048, HID), 0.1)), ctx.put_tiled(bf((HID, 24 * 256), 0.03))
+    qn, kn = ctx.put(W.normal(r, 256, 0.1)), ctx.put(W.normal(r, 256, 0.1))
+    x = W.normal(r, (T, HID))
+
+    def run(chunks):
+        kc, vc = ctx.put(np.zeros((4, 256, 256), np.uint16)), ctx.put(np.zeros((4, 8, 256, 32), np.uint16))
+        for p0, n in chunks:
+            xb, ob = ctx.put(np.ascontiguousarray(x[p0:p0 + n])), ctx.buf(n * HID * 4)
+            d = L.GqaLayerPrefillDesc(1, n, 24, 4, 256, HID, 64, 1e7, 1.0, 256, p0, 0, xb.ptr, wq.ptr, wo.ptr, qn.ptr,
+                                      kn.ptr, kc.ptr, vc.ptr, ob.ptr)
+            L.check(L.lib().vx27_hip_gqa_layer_prefill(ctx.h, C.byref(d)), "gqa_layer_prefill")
+            o = ob.download((n, HID), np.float32)
+            xb.free(), ob.free()
+        res = kc.download((4, 256, 256), np.uint16), vc.download((4, 8, 256, 32), np.uint16), o
+        kc.free(), vc.free()
+        return res
+
+    kc, vc, _ = run([(0, T)])
+    k1, v1, _ = run([(p, 1) for p in range(0, T)] if T < 100 else [(p, min(33, T - p)) for p in range(0, T, 33)])
+    assert np.array_equal(kc, k1) and np.array_equal(vc, v1)

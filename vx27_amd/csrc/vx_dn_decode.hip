@@ -260,7 +260,7 @@ __global__ __launch_bounds__(HD / CS * R) void dn_decode_kernel(DnArgs a) {
         }
         if (v_lane) {
             if (a.out) a.out[sb * a.out_tok + (size_t)vh * HD + col] = of;
-            if (a.out_packed) vx_pack_store(a.out_packed, a.B, b, vh * HD + col, of);
+            if (a.out_packed) vx_pack_store(a.out_packed, a.B, a.out_tiles, b, vh * HD + col, of);
         }
     }
 
@@ -533,8 +533,8 @@ __global__ __launch_bounds__(512) void dn_step_kernel(DnArgs a) {
         a.out[(size_t)b * a.b_step * a.out_tok + (size_t)vh * HD + lane + 64] = f1;
     }
     if (a.out_packed) {
-        vx_pack_store(a.out_packed, a.B, b, vh * HD + lane, f0);
-        vx_pack_store(a.out_packed, a.B, b, vh * HD + lane + 64, f1);
+        vx_pack_store(a.out_packed, a.B, a.out_tiles, b, vh * HD + lane, f0);
+        vx_pack_store(a.out_packed, a.B, a.out_tiles, b, vh * HD + lane + 64, f1);
     }
 }
 
@@ -711,7 +711,7 @@ __global__ __launch_bounds__(128) void dn_step_split(DnArgs a) {
         const float f = (float)(s_red[0][tid] + s_red[1][tid]);
         const int j = slice * NCOL + tid;
         if (a.out) a.out[(size_t)b * a.b_step * a.out_tok + (size_t)vh * HD + j] = f;
-        if (a.out_packed) vx_pack_store(a.out_packed, a.B, b, vh * HD + j, f);
+        if (a.out_packed) vx_pack_store(a.out_packed, a.B, a.out_tiles, b, vh * HD + j, f);
     }
 }
 
@@ -729,7 +729,7 @@ __global__ __launch_bounds__(HD) void dn_out_gate(DnArgs a) {
     const float zz = a.z[(size_t)b * a.b_step * a.z_tok + (size_t)vh * HD + col];
     of = ((of * is) * a.norm_w[col]) * silu_f(zz);
     if (a.out) a.out[(size_t)b * a.b_step * a.out_tok + (size_t)vh * HD + col] = of;
-    if (a.out_packed) vx_pack_store(a.out_packed, a.B, b, vh * HD + col, of);
+    if (a.out_packed) vx_pack_store(a.out_packed, a.B, a.out_tiles, b, vh * HD + col, of);
 }
 
 // Channel-parallel causal conv over `steps` tokens: one thread per (b, c),

@@ -26,27 +26,21 @@ __host__ __device__ __forceinline__ int vx_pass_groups(int B, int b0) {
     const int g = (B - b0 + VX_PACK_GV - 1) / VX_PACK_GV;
     return vx_round_groups(g < VX_PASS_G ? g : VX_PASS_G);
 }
-size_t vx_pack_bytes(int K, int B);
+// The token layout (tok) holds 16 vectors a tile, each part a tile of its own
+// (vx_gemv_tok.h): [K/32][ceil(B/16)][3 parts][64 lanes][8] bf16, lane (g, n)
+// of block j: vector 16 j + n, k 8g .. 8g+7.
+// The wide input projections take it from 36 vectors (8 operand groups, padded
+// to 10: their whole-K workgroups no longer fit one round of CUs: in_proj at 64
+// vectors 93 against 70 us, GQA qkv at 40 49 against 42); the narrow output
+// projections, whose whole-K grid fits one round at any group count (36 us
+// against 40 at 64 vectors), where the groups would need a second pass over
+// the weights.
+constexpr int VX_TOK_IN = 36, VX_TOK_OUT = VX_PASS_G * VX_PACK_GV + 1;
+__host__ __device__ __forceinline__ bool vx_tok_in(int B) { return B >= VX_TOK_IN; }
+__host__ __device__ __forceinline__ bool vx_tok_out(int B) { return B >= VX_TOK_OUT; }
+size_t vx_pack_bytes(int K, int B, bool tok);
 // x [B][K] (row stride x_stride) -> packed MFMA B operand (three bf16 parts).
-int vx_pack(vx27_hip_ctx *ctx, const float *x, size_t x_stride, int B, int K, uint16_t *packed);
-// y[b*y_stride + n] = sum over k of W[n][k] x_b[k] for tiled W and a packed x
-// of B vectors (one pass over W for up to 65 vectors; passes of 13 groups
-// beyond).  Each row's sum order is the same for any B.  y_zeroed: y holds
-// zeros (written by an earlier kernel on the stream), so the rows may be
-// added in two halves.
-int vx_gemv_store(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const uint16_t *packed, int B, float *y,
-                  size_t y_stride, bool y_zeroed = false);
-
-// The projection of R tokens at once (vx_gemm.hip): y[r][n] = sum over k of
-// W[n][k] x_r[k] for tiled W, fp32 x rows (x as two bf16 parts; K % 64 == 0,
-// 16-byte aligned rows).
-// ws: vx_gemm_ws_bytes of device scratch (the tokens packed for the MFMAs,
-// and the partial sums of a last round of tiles split along k)
-int vx_gemm_store(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const float *x, size_t x_stride, int R,
-                  float *y, size_t y_stride, void *ws);
-size_t vx_gemm_ws_bytes(int N, int K, int R, int n_cu);
-// whether vx_gemm_store takes this shape (else the GEMV passes)
-bool vx_gemm_fits(int N, int K, int R, const float *x, size_t x_stride, const float *y, size_t y_stride);
+int vx_pack(vx27_hip_ctx *ctx, const float *x, size_t x_stride, int B, int K, bool tok, uint16_t *packed);
 // Output in segments: rows n >= 16 rb0 of segment s (up to the next
 // segment's) go to p[r * stride + n - 16 rb0], as fp32 or as bf16 (round to
 // nearest even, vx_f32_to_bf16).  Segment 0 starts at rb0 = 0.
@@ -60,6 +54,28 @@ struct GemmOut {
     int n;
     GemmSeg s[VX_GEMM_SEGS];
 };
+// y_b[n] = sum over k of W[n][k] x_b[k] for tiled W and a packed x of B
+// vectors into output segments (operand groups: one pass over W for up to 65
+// vectors, passes of 13 groups beyond; tok: token tiles).  Each row's sum order
+// is the same for any B and either layout.  zeroed: the output (fp32) holds
+// zeros, written by an earlier kernel on the stream, so the rows may be added
+// in two halves.
+int vx_gemv_store_seg(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const uint16_t *packed, int B, bool tok,
+                      const GemmOut &out, bool zeroed = false);
+// the same to y[b*y_stride + n]
+int vx_gemv_store(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const uint16_t *packed, int B, bool tok,
+                  float *y, size_t y_stride, bool zeroed = false);
+
+// The projection of R tokens at once (vx_gemm.hip): y[r][n] = sum over k of
+// W[n][k] x_r[k] for tiled W, fp32 x rows (x as two bf16 parts; K % 64 == 0,
+// 16-byte aligned rows).
+// ws: vx_gemm_ws_bytes of device scratch (the tokens packed for the MFMAs,
+// and the partial sums of a last round of tiles split along k)
+int vx_gemm_store(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const float *x, size_t x_stride, int R,
+                  float *y, size_t y_stride, void *ws);
+size_t vx_gemm_ws_bytes(int N, int K, int R, int n_cu);
+// whether vx_gemm_store takes this shape (else the GEMV passes)
+bool vx_gemm_fits(int N, int K, int R, const float *x, size_t x_stride, const float *y, size_t y_stride);
 int vx_gemm_store_seg(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const float *x, size_t x_stride, int R,
                       const GemmOut &out, void *ws);
 bool vx_gemm_fits_seg(int N, int K, int R, const float *x, size_t x_stride, const GemmOut &out);
@@ -95,16 +111,23 @@ __device__ __forceinline__ uint16_t vx_bf16_part(float x, int p) {
 
 // Element k of vector b (of B) as the three parts of the packed operand:
 // group j = b / 5 holds its Bj <= 5 vectors' part p of vector b' at column
-// p*Bj + b'.
-__device__ __forceinline__ void vx_pack_store(uint16_t *packed, int B, int b, int k, float x) {
-    const int G = vx_pack_groups(B), j = b / VX_PACK_GV, bl = b - VX_PACK_GV * j;
-    const int Bj = min(VX_PACK_GV, B - VX_PACK_GV * j);
-    const size_t base = (((size_t)(k >> 5) * G + j) * 64 + ((k >> 3) & 3) * 16) * 8 + (k & 7);
+// p*Bj + b' (token layout: tile p of token block b / 16 at column b % 16).
+__device__ __forceinline__ void vx_pack_store(uint16_t *packed, int B, bool tok, int b, int k, float x) {
+    size_t base;   // of part 0
+    int step;      // elements between parts
+    if (tok) {
+        base = (((size_t)(k >> 5) * ((B + 15) >> 4) + (b >> 4)) * 3 * 64 + ((k >> 3) & 3) * 16 + (b & 15)) * 8 + (k & 7);
+        step = 512;
+    } else {
+        const int G = vx_pack_groups(B), j = b / VX_PACK_GV, bl = b - VX_PACK_GV * j;
+        base = (((size_t)(k >> 5) * G + j) * 64 + ((k >> 3) & 3) * 16 + bl) * 8 + (k & 7);
+        step = min(VX_PACK_GV, B - VX_PACK_GV * j) * 8;
+    }
     uint16_t h = vx_f32_to_bf16(x);
-    packed[base + (size_t)bl * 8] = h;
+    packed[base] = h;
     x = x - vx_bf16_to_f32(h);
     h = vx_f32_to_bf16(x);
-    packed[base + (size_t)(Bj + bl) * 8] = h;
+    packed[base + step] = h;
     x = x - vx_bf16_to_f32(h);
-    packed[base + (size_t)(2 * Bj + bl) * 8] = vx_f32_to_bf16(x);
+    packed[base + 2 * step] = vx_f32_to_bf16(x);
 }

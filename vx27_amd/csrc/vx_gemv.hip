@@ -26,13 +26,15 @@
 //                       k-step are adjacent (a 1 MiB slab for N = 16K rows)
 //                       (vx27_hip_pack_weights_bf16 converts row-major W)
 //
-// Both layouts go through gemv_wk_store (vx_gemv_body.h): whole-K
+// More vectors than fit a few groups go in token tiles instead
+// (vx_gemv_tok.h), with the same products and sums.  Both weight layouts go
+// through gemv_wk_store (vx_gemv_body.h) below that: whole-K
 // workgroups with the wave partials reduced in LDS, reading the weights once
 // for up to 65 vectors.  Row-major weights (the plain vx27_hip_gemv_bf16
 // call) are read as 16 rows x 64 bytes per tile.
 #include <algorithm>
 
-#include "vx_gemv_body.h"
+#include "vx_gemv_tok.h"
 
 namespace {
 
@@ -57,6 +59,28 @@ __global__ __launch_bounds__(64) void pack_x(const float *x, size_t x_stride, in
     *(uint4 *)(out + (((size_t)s * gridDim.y + j) * 64 + lane) * 8) = w;
 }
 
+// the token layout: grid (K/32, token blocks), block 64; lane (g,n) splits
+// its 8 elements of vector 16 j + n into the three tiles
+__global__ __launch_bounds__(64) void pack_x_tok(const float *x, size_t x_stride, int B, uint16_t *out) {
+    const int s = blockIdx.x, j = blockIdx.y, lane = threadIdx.x, g = lane >> 4, b = 16 * j + (lane & 15);
+    if (b >= B) return;   // padding columns feed unread output columns
+    const float *xr = x + (size_t)b * x_stride + 32 * s + 8 * g;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = xr[e];
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+        uint32_t w[4];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const uint16_t u = vx_f32_to_bf16(v[e]);
+            v[e] = v[e] - vx_bf16_to_f32(u);
+            w[e / 2] = e & 1 ? w[e / 2] | ((uint32_t)u << 16) : u;
+        }
+        *(uint4 *)(out + ((((size_t)s * gridDim.y + j) * 3 + p) * 64 + lane) * 8) = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+}
+
 // row-major W [N][K] -> tiled; grid (N/16, K/32), block 64
 __global__ __launch_bounds__(64) void pack_w(const uint16_t *W, int K, uint16_t *Wt) {
     const int rb = blockIdx.x, s = blockIdx.y, lane = threadIdx.x, g = lane >> 4, m = lane & 15;
@@ -70,7 +94,75 @@ __global__ __launch_bounds__(VX_WK_NW * 64) void gemv_wk_store(WkWeights wt, int
     vx_gemv_wk_body<RB, G>(wt, N, K, xp, Gt, g0, B, halves, epi);
 }
 
+// Epilogue of the token-tile form: the rows into their output segment
+// (fp32 or bf16; vec: 16-byte (bf16: 8-byte) aligned).
+struct TokStore {
+    GemmOut out;
+    int vec;
+    struct Pre {};
+    __device__ __forceinline__ void begin() const {}
+    __device__ __forceinline__ Pre load(int, int) const { return {}; }
+    __device__ __forceinline__ void store(int n, int b, vx_floatx4_t y, const Pre &) const {
+        GemmSeg sg = out.s[0];
+#pragma unroll
+        for (int t = 1; t < VX_GEMM_SEGS; t++)
+            if (t < out.n && n >= 16 * out.s[t].rb0) sg = out.s[t];
+        const size_t o = (size_t)b * sg.stride + (n - 16 * sg.rb0);
+        if (sg.bf16) {
+            uint16_t *yp = (uint16_t *)sg.p + o;
+            uint32_t h[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) h[e] = vx_f32_to_bf16(y[e]);
+            if (vec) *(uint2 *)yp = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+            else
+#pragma unroll
+                for (int e = 0; e < 4; e++) yp[e] = (uint16_t)h[e];
+        } else {
+            float *yp = (float *)sg.p + o;
+            if (vec) *(vx_floatx4_t *)yp = y;
+            else
+#pragma unroll
+                for (int e = 0; e < 4; e++) yp[e] = y[e];
+        }
+    }
+};
+
+template <int RB>
+__global__ __launch_bounds__(512) void gemv_tok_store(TtArgs a, TokStore epi) {
+    vx_gemv_tok_body<RB>(a, epi);
+}
+
+int gemv_tok(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const uint16_t *packed, int B, const GemmOut &out) {
+    bool vec = true;   // every segment takes 16-byte (bf16: 8-byte) stores
+    for (int q = 0; q < out.n; q++)
+        vec = vec && out.s[q].stride % 4 == 0 && ((uintptr_t)out.s[q].p & (out.s[q].bf16 ? 7 : 15)) == 0;
+    const TtPlan p = vx_gemv_tok_plan(W, packed, N, K, B, ctx->n_cu);
+    VX_TT_DISPATCH(ctx, gemv_tok_store, p, (TokStore{out, vec}));
+    return 0;
+}
+
 }  // namespace
+
+TtPlan vx_gemv_tok_plan(const uint16_t *W, const uint16_t *xp, int N, int K, int B, int n_cu) {
+    TtPlan p = {};
+    TtArgs &a = p.a;
+    a.W = W; a.xp = xp; a.N = N; a.K = K; a.B = B;
+    a.n_tt = (B + VX_TT_B - 1) / VX_TT_B;
+    const int nb = N / 16;
+    double best = 0.0;
+    for (int rb = 1; rb <= VX_TT_MAX_RB; rb++) {
+        const int tiles = (nb + rb - 1) / rb * a.n_tt;
+        const double t = (double)((tiles + n_cu - 1) / n_cu) * (0.36 + 0.055 * rb);
+        if (p.rb == 0 || t < best) {
+            best = t;
+            p.rb = rb;
+            a.n_tiles = tiles;
+        }
+    }
+    a.per_xcd = (a.n_tiles + 7) / 8;
+    p.grid = 8 * a.per_xcd;
+    return p;
+}
 
 WkPlan vx_gemv_wk_plan(int N, int K, int n_cu, int G, bool allow_halves) {
     (void)K;
@@ -95,28 +187,38 @@ WkPlan vx_gemv_wk_plan(int N, int K, int n_cu, int G, bool allow_halves) {
     return best;
 }
 
-int vx_gemv_store(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const uint16_t *packed, int B, float *y,
-                  size_t y_stride, bool y_zeroed) {
+int vx_gemv_store_seg(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const uint16_t *packed, int B, bool tok,
+                      const GemmOut &out, bool zeroed) {
     VX_REQUIRE(N > 0 && N % 16 == 0 && K > 0 && K % 32 == 0 && B >= 1,
                "gemv: N must be a multiple of 16, K of 32, B >= 1 (N=%d K=%d B=%d)", N, K, B);
+    if (tok) return gemv_tok(ctx, W, N, K, packed, B, out);
     const int Gt = vx_pack_groups(B);
     for (int g0 = 0; g0 < Gt; g0 += VX_PASS_G) {   // one pass up to 13 groups (65 vectors)
         const int b0 = g0 * VX_PACK_GV, G = vx_pass_groups(B, b0);
         const int Bp = std::min(B - b0, G * VX_PACK_GV);
-        const WkPlan p = vx_gemv_wk_plan(N, K, ctx->n_cu, G, y_zeroed);
+        const WkPlan p = vx_gemv_wk_plan(N, K, ctx->n_cu, G, zeroed);
         VX_WK_DISPATCH(ctx, gemv_wk_store, p, (WkWeights{W, 0}), N, K, packed, Gt, g0, Bp, p.halves,
-                       (WkStore{y, y_stride, b0}));
+                       (WkStore{out, b0}));
     }
     return 0;
 }
 
-size_t vx_pack_bytes(int K, int B) {
+int vx_gemv_store(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const uint16_t *packed, int B, bool tok,
+                  float *y, size_t y_stride, bool zeroed) {
+    return vx_gemv_store_seg(ctx, W, N, K, packed, B, tok, vx_gemm_out1(y, y_stride), zeroed);
+}
+
+size_t vx_pack_bytes(int K, int B, bool tok) {
+    if (tok) return (size_t)(K / 32) * ((B + 15) / 16) * 3 * 1024;
     return (size_t)(K / 32) * vx_pack_groups(B) * 64 * 8 * sizeof(uint16_t);
 }
 
-int vx_pack(vx27_hip_ctx *ctx, const float *x, size_t x_stride, int B, int K, uint16_t *packed) {
+int vx_pack(vx27_hip_ctx *ctx, const float *x, size_t x_stride, int B, int K, bool tok, uint16_t *packed) {
     VX_REQUIRE(B >= 1 && K % 32 == 0, "pack: need B >= 1, K %% 32 == 0");
-    VX_LAUNCH(ctx, pack_x, dim3(K / 32, vx_pack_groups(B)), dim3(64), x, x_stride, B, packed);
+    if (tok)
+        VX_LAUNCH(ctx, pack_x_tok, dim3(K / 32, (B + 15) / 16), dim3(64), x, x_stride, B, packed);
+    else
+        VX_LAUNCH(ctx, pack_x, dim3(K / 32, vx_pack_groups(B)), dim3(64), x, x_stride, B, packed);
     return 0;
 }
 
@@ -139,14 +241,15 @@ extern "C" int vx27_hip_gemv_bf16(vx27_hip_ctx *ctx, const uint16_t *W, int N, i
     // one pass over W per 13 groups (65 vectors), each packing its vectors
     const int Bp0 = std::min(B, VX_PASS_G * VX_PACK_GV);
     void *scr;
-    if (vx_ctx_scratch(ctx, vx_pack_bytes(K, Bp0), &scr)) return -1;
+    // (row-major weights go through the whole-K form at any B: operand groups)
+    if (vx_ctx_scratch(ctx, vx_pack_bytes(K, Bp0, false), &scr)) return -1;
     uint16_t *packed = (uint16_t *)scr;
     for (int b0 = 0; b0 < B; b0 += VX_PASS_G * VX_PACK_GV) {
         const int Bp = std::min(B - b0, VX_PASS_G * VX_PACK_GV), G = vx_pack_groups(Bp);
-        if (vx_pack(ctx, x + (size_t)b0 * x_stride, x_stride, Bp, K, packed)) return -1;
+        if (vx_pack(ctx, x + (size_t)b0 * x_stride, x_stride, Bp, K, false, packed)) return -1;
         const WkPlan p = vx_gemv_wk_plan(N, K, ctx->n_cu, G);
         VX_WK_DISPATCH(ctx, gemv_wk_store, p, (WkWeights{W, 1}), N, K, packed, G, 0, Bp, p.halves,
-                       (WkStore{y, y_stride, b0}));
+                       (WkStore{vx_gemm_out1(y, y_stride), b0}));
     }
     return 0;
 }

@@ -191,24 +191,37 @@ __device__ __forceinline__ void vx_gemv_wk_body(const WkWeights &wt, int N, int 
     epi(row0, rows, WkRows<RB, G>{ct, B, nh}, tid, pre);
 }
 
-// Epilogue: y[(b0 + b)*y_stride + n] for every row n of the workgroup
-// (added with an atomic in a half workgroup: y must then start at zero).
+// Epilogue: row n of vector b0 + b into the output segment that holds row n
+// (added with an atomic in a half workgroup: the output, fp32, must then
+// start at zero).
 struct WkStore {
-    float *y;
-    size_t y_stride;
+    GemmOut out;
     int b0;
     struct Pre {};
     __device__ __forceinline__ Pre prefetch(int, int, int) const { return {}; }
     template <int RB, int G>
     __device__ __forceinline__ void operator()(int row0, int rows, const WkRows<RB, G> &c, int tid, const Pre &) const {
         for (int t = tid; t < rows * c.B; t += c.nh * 4 * 64) {
-            const int r = t % rows, b = t / rows;
-            float *yp = y + (size_t)(b0 + b) * y_stride + row0 + r;
-            if (c.nh == 1) atomicAdd(yp, c.y(r, b));
-            else *yp = c.y(r, b);
+            const int r = t % rows, b = t / rows, n = row0 + r;
+            GemmSeg sg = out.s[0];
+            if (out.n > 1)
+#pragma unroll
+                for (int q = 1; q < VX_GEMM_SEGS; q++)
+                    if (q < out.n && n >= 16 * out.s[q].rb0) sg = out.s[q];
+            const size_t o = (size_t)(b0 + b) * sg.stride + (n - 16 * sg.rb0);
+            if (sg.bf16) ((uint16_t *)sg.p)[o] = vx_f32_to_bf16(c.y(r, b));
+            else if (c.nh == 1) atomicAdd((float *)sg.p + o, c.y(r, b));
+            else ((float *)sg.p)[o] = c.y(r, b);
         }
     }
 };
+// one fp32 segment
+static inline GemmOut vx_gemm_out1(float *y, size_t stride) {
+    GemmOut o = {};
+    o.n = 1;
+    o.s[0] = GemmSeg{0, 0, stride, y};
+    return o;
+}
 
 // Launch plan for an N x K matrix and a pass of G groups: RB row blocks per
 // workgroup, whole (halves = 1, grid ceil(N / 16 RB)) or split in two half

@@ -283,6 +283,7 @@ struct CombArgs {
     size_t g_ss, g_hs;
     float *out;                  // [B][n_q][256] or NULL
     uint16_t *out_packed;        // optional packed GEMV operand of out (K = n_q*256)
+    bool tok;                    // (in the token layout)
     float *zero;                 // optional: zero_n floats cleared (the next projection's output)
     size_t zero_n;
 };
@@ -365,7 +366,7 @@ __global__ __launch_bounds__(1024) void gqa_combine(CombArgs a) {
             r = r * (1.0f / (1.0f + expf(-gl)));
         }
         if (a.out) a.out[((size_t)b * a.n_q + h) * HDG + d] = r;
-        if (a.out_packed) vx_pack_store(a.out_packed, a.B, b, h * HDG + d, r);
+        if (a.out_packed) vx_pack_store(a.out_packed, a.B, a.tok, b, h * HDG + d, r);
     }
 }
 
@@ -455,7 +456,7 @@ size_t vx_gqa_scratch_bytes(const vx27_gqa_desc *d) {
 // The decode step with caller-provided scratch of vx_gqa_scratch_bytes(d);
 // out_packed (optional) receives the output as the packed GEMV operand;
 // zero (optional) is cleared by the combine kernel.
-int vx_gqa_decode_into(vx27_hip_ctx *ctx, const vx27_gqa_desc *d, void *scr, uint16_t *out_packed, float *zero,
+int vx_gqa_decode_into(vx27_hip_ctx *ctx, const vx27_gqa_desc *d, void *scr, uint16_t *out_packed, bool tok, float *zero,
                        size_t zero_n) {
     if (gqa_check(d)) return -1;
     RopeTab rt = {};
@@ -489,6 +490,7 @@ int vx_gqa_decode_into(vx27_hip_ctx *ctx, const vx27_gqa_desc *d, void *scr, uin
     ca.part_o = part_o; ca.part_ml = part_ml; ca.gate = (d->flags & VX27_GQA_NO_GATE) ? nullptr : d->gate;
     ca.g_ss = d->gate_seq_stride; ca.g_hs = d->gate_head_stride; ca.out = d->out;
     ca.out_packed = out_packed;
+    ca.tok = tok;
     ca.zero = zero; ca.zero_n = zero_n;
     const int cb_waves = std::min(CB_W, (n_split + CB_N - 1) / CB_N);
     VX_LAUNCH(ctx, gqa_combine, dim3(d->n_q, d->B), dim3(64 * cb_waves), ca);

@@ -22,7 +22,7 @@
 #include <algorithm>
 
 #include "vx_dn.h"
-#include "vx_gemv_body.h"
+#include "vx_gemv_tok.h"
 #include "vx_gqa.h"
 
 
@@ -177,6 +177,92 @@ __global__ __launch_bounds__(VX_WK_NW * 64) void gemv_dn_in(WkWeights wt, int N,
     vx_gemv_wk_body<RB, G>(wt, N, K, xp, Gt, g0, B, 1, epi);   // whole rows (the conv needs them)
 }
 
+// The same epilogue after the token-tile form (vx_gemv_tok.h), four rows of
+// one vector at a time (C, vd: multiples of 128, nv of 8, so four rows never
+// straddle two outputs).  vec: the conv state is 16-byte aligned.
+struct DnInTok {
+    DnInArgs a;
+    int vec;
+    struct Pre {
+        uint4 w[4];   // conv weights of the four channels (bf16: w[0..1])
+        float st[12];
+    };
+    __device__ __forceinline__ void begin() const {
+        if (!a.zero) return;   // this workgroup's share of the range to clear
+        const size_t nwg = gridDim.x, wg = blockIdx.x;
+        const size_t lo = a.zero_n * wg / nwg, hi = a.zero_n * (wg + 1) / nwg;
+        for (size_t i = lo + threadIdx.x; i < hi; i += blockDim.x) a.zero[i] = 0.0f;
+    }
+    __device__ __forceinline__ Pre load(int n, int b) const {
+        Pre p;
+        if (n >= a.C) return p;
+        if (a.conv_bf16) {
+            const uint4 *w = (const uint4 *)((const uint16_t *)a.conv_w + 4 * (size_t)n);
+            p.w[0] = w[0];
+            p.w[1] = w[1];
+        } else {
+            const uint4 *w = (const uint4 *)((const float *)a.conv_w + 4 * (size_t)n);
+#pragma unroll
+            for (int e = 0; e < 4; e++) p.w[e] = w[e];
+        }
+        const float *sp = a.conv_state + ((size_t)b * a.C + n) * 3;
+        if (vec)
+#pragma unroll
+            for (int e = 0; e < 3; e++) *(float4 *)(p.st + 4 * e) = *(const float4 *)(sp + 4 * e);
+        else
+#pragma unroll
+            for (int e = 0; e < 12; e++) p.st[e] = sp[e];
+        return p;
+    }
+    __device__ __forceinline__ void store(int n, int b, vx_floatx4_t y, const Pre &p) const {
+        if (n < a.C) {
+            float st[12], o[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float w[4];
+                if (a.conv_bf16) {
+                    const uint32_t u0 = e & 1 ? p.w[e / 2].z : p.w[e / 2].x, u1 = e & 1 ? p.w[e / 2].w : p.w[e / 2].y;
+                    w[0] = __uint_as_float(u0 << 16);
+                    w[1] = __uint_as_float(u0 & 0xffff0000u);
+                    w[2] = __uint_as_float(u1 << 16);
+                    w[3] = __uint_as_float(u1 & 0xffff0000u);
+                } else {
+                    w[0] = __uint_as_float(p.w[e].x);
+                    w[1] = __uint_as_float(p.w[e].y);
+                    w[2] = __uint_as_float(p.w[e].z);
+                    w[3] = __uint_as_float(p.w[e].w);
+                }
+                float c[3] = {p.st[3 * e], p.st[3 * e + 1], p.st[3 * e + 2]};
+                o[e] = conv_step(c, w, y[e]);
+                st[3 * e] = c[0];
+                st[3 * e + 1] = c[1];
+                st[3 * e + 2] = c[2];
+            }
+            *(float4 *)(a.act + (size_t)b * a.C + n) = make_float4(o[0], o[1], o[2], o[3]);
+            float *sp = a.conv_state + ((size_t)b * a.C + n) * 3;
+            if (vec)
+#pragma unroll
+                for (int e = 0; e < 3; e++) *(float4 *)(sp + 4 * e) = *(const float4 *)(st + 4 * e);
+            else
+#pragma unroll
+                for (int e = 0; e < 12; e++) sp[e] = st[e];
+            return;
+        }
+        int r = n - a.C;
+        float *o = a.z + (size_t)b * a.vd + r;
+        if (r >= a.vd) {
+            r -= a.vd;
+            o = (r < a.nv ? a.ga + r : a.gb + (r - a.nv)) + (size_t)b * a.nv;
+        }
+        *(vx_floatx4_t *)o = y;
+    }
+};
+
+template <int RB>
+__global__ __launch_bounds__(512) void gemv_dn_in_tok(TtArgs a, DnInTok epi) {
+    vx_gemv_tok_body<RB>(a, epi);
+}
+
 __global__ void advance_pos_kernel(int *pos, int B) {
     const int b = threadIdx.x;
     if (b < B) pos[b] += 1;
@@ -220,12 +306,14 @@ __global__ __launch_bounds__(256) void qkv_to_bf16(const float *y, int Nq, int k
 
 }  // namespace
 
-extern "C" size_t vx27_hip_pack_bytes(int K, int B) { return vx_pack_bytes(K, B); }
+extern "C" size_t vx27_hip_pack_bytes(int K, int B) {
+    return vx_pack_bytes(K, B, vx_tok_in(B));
+}
 
 extern "C" int vx27_hip_pack_x(vx27_hip_ctx *ctx, const float *x, int B, int K, uint16_t *packed) {
     if (vx_ctx_enter(ctx)) return -1;
     VX_REQUIRE(x && packed && B >= 1, "vx27_hip_pack_x: bad arguments");
-    return vx_pack(ctx, x, (size_t)K, B, K, packed);
+    return vx_pack(ctx, x, (size_t)K, B, K, vx_tok_in(B), packed);
 }
 
 extern "C" int vx27_hip_dn_layer_decode(vx27_hip_ctx *ctx, const vx27_dn_layer_desc *d) {
@@ -244,11 +332,12 @@ extern "C" int vx27_hip_dn_layer_decode(vx27_hip_ctx *ctx, const vx27_dn_layer_d
     VX_REQUIRE(((uintptr_t)d->conv_w & 15) == 0, "vx27_hip_dn_layer_decode: conv_w must be 16-byte aligned");
     const int B = d->B, nv = d->nv, qd = d->nqk * HD, vd = nv * HD, C = 2 * qd + vd, H = d->hidden;
     const int Nin = C + vd + 2 * nv;
-    const size_t pk_x = d->x_packed ? 0 : align256(vx_pack_bytes(H, B));
+    const bool tok_in = vx_tok_in(B), tok_out = vx_tok_out(B);
+    const size_t pk_x = d->x_packed ? 0 : align256(vx_pack_bytes(H, B, tok_in));
     const size_t act_b = align256((size_t)B * C * 4), z_b = align256((size_t)B * vd * 4);
     const size_t g_b = align256((size_t)B * nv * sizeof(float));
     const size_t gm_b = align256((size_t)B * nv * sizeof(double2));
-    const size_t pk_o = align256(vx_pack_bytes(vd, B));
+    const size_t pk_o = align256(vx_pack_bytes(vd, B, tok_out));
     void *scr;
     if (vx_ctx_scratch(ctx, pk_x + act_b + z_b + 2 * g_b + gm_b + pk_o, &scr)) return -1;
     char *p = (char *)scr;
@@ -261,8 +350,14 @@ extern "C" int vx27_hip_dn_layer_decode(vx27_hip_ctx *ctx, const vx27_dn_layer_d
     double2 *gates = (double2 *)p; p += gm_b;
     uint16_t *op = (uint16_t *)p;
 
-    if (!d->x_packed && vx_pack(ctx, d->x, (size_t)H, B, H, xp)) return -1;
-    const int Gt = vx_pack_groups(B);
+    if (!d->x_packed && vx_pack(ctx, d->x, (size_t)H, B, H, tok_in, xp)) return -1;
+    if (tok_in) {
+        const DnInArgs ea = {B, C, vd, nv, d->conv_state, d->conv_w, d->conv_w_dtype == VX27_BF16, act, z, ga, gb,
+                             0, tok_out ? nullptr : d->out, (size_t)B * H};
+        const TtPlan p = vx_gemv_tok_plan(d->w_in, xp, Nin, H, B, ctx->n_cu);
+        VX_TT_DISPATCH(ctx, gemv_dn_in_tok, p, (DnInTok{ea, ((uintptr_t)d->conv_state & 15) == 0}));
+    }
+    const int Gt = tok_in ? 0 : vx_pack_groups(B);
     for (int g0 = 0; g0 < Gt; g0 += VX_PASS_G) {   // one pass over W_in up to 13 groups (65 vectors)
         const int b0 = g0 * VX_PACK_GV, G = vx_pass_groups(B, b0);
         const int Bp = B - b0 < G * VX_PACK_GV ? B - b0 : G * VX_PACK_GV;
@@ -282,14 +377,14 @@ extern "C" int vx27_hip_dn_layer_decode(vx27_hip_ctx *ctx, const vx27_dn_layer_d
     ra.q_tok = ra.k_tok = ra.v_tok = (size_t)C;
     ra.ga = ga; ra.gb = gb; ra.A_log = d->A_log; ra.dt_bias = d->dt_bias;   // mapped by the step kernel
     ra.norm_w = d->norm_w; ra.z = z; ra.z_tok = (size_t)vd;
-    ra.out = nullptr; ra.out_tok = (size_t)vd; ra.out_packed = op;
+    ra.out = nullptr; ra.out_tok = (size_t)vd; ra.out_packed = op; ra.out_tiles = tok_out;
     if (!vx_dn_single_step(ra)) {   // (the multi-step kernel takes mapped gates)
         if (vx_dn_gates(ctx, (size_t)B * nv, nv, ga, gb, d->A_log, d->dt_bias, gates)) return -1;
         ra.gates = gates;
     }
     if (vx_dn_recurrence(ctx, ra)) return -1;
 
-    return vx_gemv_store(ctx, d->w_out, H, vd, op, B, d->out, (size_t)H, true);
+    return vx_gemv_store(ctx, d->w_out, H, vd, op, B, tok_out, d->out, (size_t)H, true);
 }
 
 extern "C" int vx27_hip_gqa_layer_decode(vx27_hip_ctx *ctx, const vx27_gqa_layer_desc *d) {
@@ -311,9 +406,10 @@ extern "C" int vx27_hip_gqa_layer_decode(vx27_hip_ctx *ctx, const vx27_gqa_layer
     g.q_norm_w = d->q_norm_w; g.k_norm_w = d->k_norm_w;
     g.k_cache = d->k_cache; g.v_cache = d->v_cache; g.n_split = d->n_split;
 
-    const size_t pk_x = d->x_packed ? 0 : align256(vx_pack_bytes(H, B));
+    const bool tok_in = vx_tok_in(B), tok_out = vx_tok_out(B);
+    const size_t pk_x = d->x_packed ? 0 : align256(vx_pack_bytes(H, B, tok_in));
     const size_t y_b = align256((size_t)B * Nqkv * 4);
-    const size_t pk_a = align256(vx_pack_bytes(Ka, B));
+    const size_t pk_a = align256(vx_pack_bytes(Ka, B, tok_out));
     // placeholders so the scratch size of the attention step can be planned
     g.q = g.gate = g.k_new = g.v_new = (const float *)1;
     const size_t gq_b = align256(vx_gqa_scratch_bytes(&g));
@@ -326,13 +422,13 @@ extern "C" int vx27_hip_gqa_layer_decode(vx27_hip_ctx *ctx, const vx27_gqa_layer
     uint16_t *ap = (uint16_t *)p; p += pk_a;
     void *gscr = p;
 
-    if (!d->x_packed && vx_pack(ctx, d->x, (size_t)H, B, H, xp)) return -1;
-    if (vx_gemv_store(ctx, d->w_qkv, Nqkv, H, xp, B, y, (size_t)Nqkv)) return -1;
+    if (!d->x_packed && vx_pack(ctx, d->x, (size_t)H, B, H, tok_in, xp)) return -1;
+    if (vx_gemv_store(ctx, d->w_qkv, Nqkv, H, xp, B, tok_in, y, (size_t)Nqkv)) return -1;
     g.q = y; g.gate = y + hd; g.k_new = y + Nq; g.v_new = y + Nq + (size_t)d->n_kv * hd;
     g.out = nullptr;
     // the combine kernel clears out for o_proj's two halves
-    if (vx_gqa_decode_into(ctx, &g, gscr, ap, d->out, (size_t)B * H)) return -1;
-    return vx_gemv_store(ctx, d->w_o, H, Ka, ap, B, d->out, (size_t)H, true);
+    if (vx_gqa_decode_into(ctx, &g, gscr, ap, tok_out, d->out, (size_t)B * H)) return -1;
+    return vx_gemv_store(ctx, d->w_o, H, Ka, ap, B, tok_out, d->out, (size_t)H, true);
 }
 
 extern "C" int vx27_hip_advance_pos(vx27_hip_ctx *ctx, int *pos, int B) {
@@ -380,10 +476,11 @@ extern "C" int vx27_hip_dn_layer_prefill(vx27_hip_ctx *ctx, const vx27_dn_layer_
     pd.S = d->S; pd.A_log = d->A_log; pd.dt_bias = d->dt_bias;
     pd.conv_state = d->conv_state; pd.conv_w = d->conv_w; pd.conv_w_dtype = d->conv_w_dtype;
     pd.norm_w = d->norm_w; pd.S_ckpt = d->S_ckpt; pd.conv_ckpt = d->conv_ckpt;
-    const size_t pk_x = align256(vx_pack_bytes(H, R)), y_b = align256((size_t)R * Nin * 4);
+    const bool tok_in = vx_tok_in(R), tok_out = vx_tok_out(R);
+    const size_t pk_x = align256(vx_pack_bytes(H, R, tok_in)), y_b = align256((size_t)R * Nin * 4);
     const size_t x_b = align256((size_t)R * C * 4), z_b = align256((size_t)R * vd * 4);
     const size_t g_b = align256((size_t)R * nv * 4), o_b = align256((size_t)R * vd * 4);
-    const size_t pk_o = align256(vx_pack_bytes(vd, R));
+    const size_t pk_o = align256(vx_pack_bytes(vd, R, tok_out));
     const size_t inner = vx_dn_prefill_scratch(&pd);
     // [qkv | z | a | b] = W_in x for all B*T tokens: a long prompt of the
     // chunked form in the GEMM (W_in read once per 256 tokens, x as two bf16
@@ -417,12 +514,15 @@ extern "C" int vx27_hip_dn_layer_prefill(vx27_hip_ctx *ctx, const vx27_dn_layer_
     seg.s[3] = GemmSeg{(C + vd + nv) / 16, 0, (size_t)nv, gb};
     if (gemm && nv % 16 == 0 && vx_gemm_fits_seg(Nin, H, R, d->x, (size_t)H, seg)) {
         if (vx_gemm_store_seg(ctx, d->w_in, Nin, H, d->x, (size_t)H, R, seg, gws)) return -1;
+    } else if (!gemm && nv % 16 == 0) {
+        if (vx_pack(ctx, d->x, (size_t)H, R, H, tok_in, xp)) return -1;
+        if (vx_gemv_store_seg(ctx, d->w_in, Nin, H, xp, R, tok_in, seg)) return -1;
     } else {
         if (gemm && vx_gemm_fits(Nin, H, R, d->x, (size_t)H, y, (size_t)Nin)) {
             if (vx_gemm_store(ctx, d->w_in, Nin, H, d->x, (size_t)H, R, y, (size_t)Nin, gws)) return -1;
         } else {
-            if (vx_pack(ctx, d->x, (size_t)H, R, H, xp)) return -1;
-            if (vx_gemv_store(ctx, d->w_in, Nin, H, xp, R, y, (size_t)Nin)) return -1;
+            if (vx_pack(ctx, d->x, (size_t)H, R, H, tok_in, xp)) return -1;
+            if (vx_gemv_store(ctx, d->w_in, Nin, H, xp, R, tok_in, y, (size_t)Nin)) return -1;
         }
         const size_t ys = (size_t)Nin * 4;
         VX_HIP(hipMemcpy2DAsync(xq, (size_t)C * 4, y, ys, (size_t)C * 4, (size_t)R, hipMemcpyDeviceToDevice,
@@ -443,8 +543,8 @@ extern "C" int vx27_hip_dn_layer_prefill(vx27_hip_ctx *ctx, const vx27_dn_layer_
     const bool gemm_out = gemm && vx_gemm_fits_seg(H, vd, R, o, (size_t)vd, oseg);
     if (vx_dn_prefill_into(ctx, &pd, p, gemm_out ? opk : nullptr)) return -1;
     if (gemm_out) return vx_gemm_store_packed(ctx, d->w_out, H, vd, opk, R, oseg, gws);
-    if (vx_pack(ctx, o, (size_t)vd, R, vd, op)) return -1;
-    return vx_gemv_store(ctx, d->w_out, H, vd, op, R, d->out, (size_t)H);
+    if (vx_pack(ctx, o, (size_t)vd, R, vd, tok_out, op)) return -1;
+    return vx_gemv_store(ctx, d->w_out, H, vd, op, R, tok_out, d->out, (size_t)H);
 }
 
 extern "C" int vx27_hip_gqa_layer_prefill(vx27_hip_ctx *ctx, const vx27_gqa_layer_prefill_desc *d) {
@@ -464,9 +564,10 @@ extern "C" int vx27_hip_gqa_layer_prefill(vx27_hip_ctx *ctx, const vx27_gqa_laye
     gp.q_tok_stride = (size_t)Nq; gp.q_head_stride = (size_t)2 * hd;
     gp.gate_tok_stride = (size_t)Nq; gp.gate_head_stride = (size_t)2 * hd;
     gp.q_norm_w = d->q_norm_w; gp.k_norm_w = d->k_norm_w; gp.k_cache = d->k_cache; gp.v_cache = d->v_cache;
-    const size_t pk_x = align256(vx_pack_bytes(H, R)), y_b = align256((size_t)R * Nqkv * 4);
+    const bool tok_in = vx_tok_in(R), tok_out = vx_tok_out(R);
+    const size_t pk_x = align256(vx_pack_bytes(H, R, tok_in)), y_b = align256((size_t)R * Nqkv * 4);
     const size_t qg_b = align256((size_t)R * Nq * 2), kv_b = align256((size_t)R * kvd * 2);
-    const size_t at_b = align256((size_t)R * Ka * 4), pk_a = align256(vx_pack_bytes(Ka, R));
+    const size_t at_b = align256((size_t)R * Ka * 4), pk_a = align256(vx_pack_bytes(Ka, R, tok_out));
     const size_t inner = vx_gqa_prefill_scratch(&gp);
     // a long prompt's projections in the GEMM (weights once per 256 tokens),
     // rounded to bf16 straight into q|gate, k and v
@@ -491,9 +592,12 @@ extern "C" int vx27_hip_gqa_layer_prefill(vx27_hip_ctx *ctx, const vx27_gqa_laye
     seg.s[2] = GemmSeg{(Nq + kvd) / 16, 1, (size_t)kvd, vb};
     if (gemm && vx_gemm_fits_seg(Nqkv, H, R, d->x, (size_t)H, seg)) {
         if (vx_gemm_store_seg(ctx, d->w_qkv, Nqkv, H, d->x, (size_t)H, R, seg, gws)) return -1;
+    } else if (!gemm) {
+        if (vx_pack(ctx, d->x, (size_t)H, R, H, tok_in, xp)) return -1;
+        if (vx_gemv_store_seg(ctx, d->w_qkv, Nqkv, H, xp, R, tok_in, seg)) return -1;
     } else {
-        if (vx_pack(ctx, d->x, (size_t)H, R, H, xp)) return -1;
-        if (vx_gemv_store(ctx, d->w_qkv, Nqkv, H, xp, R, y, (size_t)Nqkv)) return -1;
+        if (vx_pack(ctx, d->x, (size_t)H, R, H, tok_in, xp)) return -1;
+        if (vx_gemv_store(ctx, d->w_qkv, Nqkv, H, xp, R, tok_in, y, (size_t)Nqkv)) return -1;
         VX_LAUNCH(ctx, qkv_to_bf16, dim3((unsigned)R, (unsigned)((Nqkv + 255) / 256)), dim3(256), y, Nq, kvd, qg, kb,
                   vb);
     }
@@ -504,6 +608,6 @@ extern "C" int vx27_hip_gqa_layer_prefill(vx27_hip_ctx *ctx, const vx27_gqa_laye
     // item's loads)
     if (gemm && vx_gemm_fits(H, Ka, R, att, (size_t)Ka, d->out, (size_t)H))
         return vx_gemm_store(ctx, d->w_o, H, Ka, att, (size_t)Ka, R, d->out, (size_t)H, gws);
-    if (vx_pack(ctx, att, (size_t)Ka, R, Ka, ap)) return -1;
-    return vx_gemv_store(ctx, d->w_o, H, Ka, ap, R, d->out, (size_t)H);
+    if (vx_pack(ctx, att, (size_t)Ka, R, Ka, tok_out, ap)) return -1;
+    return vx_gemv_store(ctx, d->w_o, H, Ka, ap, R, tok_out, d->out, (size_t)H);
 }
