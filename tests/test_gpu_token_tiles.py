@@ -1,10 +1,12 @@
 """GPU tests of the token-tile projections (batches and prompts of more
-vectors than the operand groups of one pass hold): they keep the sums of the
-single-vector calls, so every comparison is bit for bit.
+vectors than the operand groups of one pass hold) and of the checkpointed
+multi-step recurrence: both keep the sums of the single-vector, single-step
+calls, so every comparison is bit for bit.
 
 Sizes: a small layer (hidden 160: fewer k-steps than the eight classes of the
 sum; 161 row blocks: no multiple of any workgroup's), batches at the edges of
-16-vector blocks, 64-vector tiles and of both layouts' ranges."""
+16-vector blocks, 64-vector tiles and of both layouts' ranges, windows at the
+edges of the recurrence's 8-token blocks."""
 import ctypes as C
 
 import numpy as np
@@ -73,6 +75,32 @@ def test_decode_batch_bits(ctx, B, conv_bf16, skew):
         one = decode(ctx, dev, x[b:b + 1], S[b:b + 1], conv[b:b + 1])
         for g, o, n in zip(got, one, ("out", "S", "conv")):
             assert np.array_equal(g[b], o[0]), (n, b)
+
+
+@pytest.mark.parametrize("B,T", [(1, 1), (3, 2), (1, 8), (2, 9), (1, 17), (5, 7), (1, 36), (2, 33), (1, 70)])
+def test_checkpoint_window_bits(ctx, B, T):
+    """A window with checkpoints gives the bits of T decode calls."""
+    from vx27_amd import lib as L, workloads as W
+    r = W.rng(32, f"tok_window_{B}_{T}")
+    dev = weights(ctx, r)
+    _, S, conv = inputs(r, B)
+    x = W.normal(r, (B, T, HID))
+    Sd, cd, xb, ob = ctx.put(S), ctx.put(conv), ctx.put(x), ctx.buf(B * T * HID * 4)
+    sk, ck = ctx.buf(T * S.nbytes), ctx.buf(T * conv.nbytes)
+    d = L.DnLayerPrefillDesc(B, T, NQK, NV, 128, HID, 0, xb.ptr, dev["w_in"].ptr, dev["w_out"].ptr, dev["conv_w"].ptr,
+                             dev["dt"], dev["A_log"].ptr, dev["dt_bias"].ptr, dev["norm_w"].ptr, Sd.ptr, cd.ptr,
+                             ob.ptr)
+    d.S_ckpt, d.conv_ckpt = sk.ptr, ck.ptr
+    L.check(L.lib().vx27_hip_dn_layer_prefill(ctx.h, C.byref(d)), "dn_layer_prefill")
+    out = ob.download((B, T, HID), np.float32)
+    S_all, c_all = sk.download((B, T) + S.shape[1:], np.float32), ck.download((B, T) + conv.shape[1:], np.float32)
+    for t in range(T):
+        o, S, conv = decode(ctx, dev, np.ascontiguousarray(x[:, t]), S, conv)
+        assert np.array_equal(out[:, t], o) and np.array_equal(S_all[:, t], S) and np.array_equal(c_all[:, t], conv), t
+    assert np.array_equal(Sd.download(S.shape, np.float32), S)
+    assert np.array_equal(cd.download(conv.shape, np.float32), conv)
+    for b in (Sd, cd, xb, ob, sk, ck):
+        b.free()
 
 
 @pytest.mark.parametrize("T", [36, 66, 255])

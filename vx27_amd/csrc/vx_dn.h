@@ -142,6 +142,12 @@ int vx_dn_gates(vx27_hip_ctx *ctx, size_t n, int nv, const float *ga, const floa
 
 // Launch the recurrence (one or more workgroups per (sequence, value head)).
 int vx_dn_recurrence(vx27_hip_ctx *ctx, const DnArgs &a);
+// a.steps steps with the state after each written to S_ckpt
+// [B][steps][nv][128][128] too, bit-identical to single steps (q, k, v and the
+// raw gate inputs given, rows b steps + t; 16-byte aligned states:
+// vx_dn_steps_ok; out_packed: of all the rows).
+int vx_dn_steps(vx27_hip_ctx *ctx, const DnArgs &a, float *S_ckpt);
+bool vx_dn_steps_ok(const DnArgs &a, const float *S_ckpt);
 // Whether vx_dn_recurrence runs a call as one single-step kernel (which can
 // also map the gates itself, with gates == NULL).
 bool vx_dn_single_step(const DnArgs &a);
@@ -154,3 +160,8 @@ size_t vx_dn_prefill_scratch(const vx27_dn_prefill_desc *d);
 // it next; the chunked form with VX27_DN_OUT_GATE only (d->out then holds
 // the ungated output).
 int vx_dn_prefill_into(vx27_hip_ctx *ctx, const vx27_dn_prefill_desc *d, void *scr, char *out_packed = nullptr);
+// The checkpointed window with its output as the packed GEMV operand of the
+// rows instead (tok: in the token layout), for calls that
+// vx_dn_prefill_packs accepts.
+bool vx_dn_prefill_packs(const vx27_dn_prefill_desc *d);
+int vx_dn_prefill_window(vx27_hip_ctx *ctx, const vx27_dn_prefill_desc *d, void *scr, uint16_t *out_op, bool tok);

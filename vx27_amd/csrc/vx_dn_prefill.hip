@@ -2512,8 +2512,15 @@ size_t vx_dn_prefill_scratch(const vx27_dn_prefill_desc *d) {
     return al256(n_rec * (x3 ? XREC : REC)) + al256(n_rec * sizeof(float)) + glue_bytes;
 }
 
+bool vx_dn_prefill_packs(const vx27_dn_prefill_desc *d) {
+    DnArgs a = {};
+    a.S = d->S;
+    return d->S_ckpt && vx_dn_steps_ok(a, d->S_ckpt);
+}
+
 // The exact path: the decode kernels token by token (prefill layout).
-static int dn_prefill_exact(vx27_hip_ctx *ctx, const vx27_dn_prefill_desc *d, void *scr) {
+static int dn_prefill_exact(vx27_hip_ctx *ctx, const vx27_dn_prefill_desc *d, void *scr, uint16_t *out_op = nullptr,
+                            bool tok = false) {
     const int qd = d->nqk * HD, vd = d->nv * HD, C = 2 * qd + vd;
     const bool conv = (d->flags & VX27_DN_CONV) != 0;
     const size_t rows = (size_t)d->B * d->T;
@@ -2522,7 +2529,8 @@ static int dn_prefill_exact(vx27_hip_ctx *ctx, const vx27_dn_prefill_desc *d, vo
     double2 *gates = (double2 *)scr;
     float *act = (float *)((char *)scr + gate_bytes + opre_bytes);
     const size_t n_gate = rows * d->nv;
-    if (vx_dn_gates(ctx, n_gate, d->nv, d->a, d->b, d->A_log, d->dt_bias, gates)) return -1;
+    const bool window = vx_dn_prefill_packs(d);   // one launch, each token's state written out
+    if (!window && vx_dn_gates(ctx, n_gate, d->nv, d->a, d->b, d->A_log, d->dt_bias, gates)) return -1;
     if (conv) {
         ConvArgs ca = {d->B, C, d->T, d->conv_w_dtype == VX27_BF16, d->conv_state, d->conv_w, d->x, act, 1, d->T,
                        d->conv_ckpt};
@@ -2546,7 +2554,14 @@ static int dn_prefill_exact(vx27_hip_ctx *ctx, const vx27_dn_prefill_desc *d, vo
         a.qk_buf = (float *)((char *)act + al256(rows * C * sizeof(float)));
         return vx_dn_recurrence(ctx, a);
     }
-    // token by token, the state written out after each (single-step kernel)
+    if (window) {
+        a.steps = d->T;
+        a.q = act; a.k = act + qd; a.v = act + 2 * qd;
+        a.ga = d->a; a.gb = d->b; a.A_log = d->A_log; a.dt_bias = d->dt_bias;
+        a.out = out_op ? nullptr : d->out; a.out_packed = out_op; a.out_tiles = tok;
+        return vx_dn_steps(ctx, a, d->S_ckpt);
+    }
+    // token by token, the state copied out after each (single-step kernel)
     const size_t s_bytes = (size_t)d->nv * HD * HD * sizeof(float);
     for (int t = 0; t < d->T; t++) {
         DnArgs at = a;
@@ -2683,6 +2698,11 @@ int vx_dn_prefill_into(vx27_hip_ctx *ctx, const vx27_dn_prefill_desc *d, void *s
         VX_LAUNCH(ctx, dnp_out_gate, dim3((unsigned)((nrow + 31) / 32)), dim3(256), nrow, d->z, d->norm_w, d->out);
     }
     return 0;
+}
+
+int vx_dn_prefill_window(vx27_hip_ctx *ctx, const vx27_dn_prefill_desc *d, void *scr, uint16_t *out_op, bool tok) {
+    if (dn_prefill_check(d)) return -1;
+    return dn_prefill_exact(ctx, d, scr, out_op, tok);
 }
 
 extern "C" int vx27_hip_dn_prefill(vx27_hip_ctx *ctx, const vx27_dn_prefill_desc *d) {

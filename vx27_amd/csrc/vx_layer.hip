@@ -541,6 +541,10 @@ extern "C" int vx27_hip_dn_layer_prefill(vx27_hip_ctx *ctx, const vx27_dn_layer_
     oseg.n = 1;
     oseg.s[0] = GemmSeg{0, 0, (size_t)H, d->out};
     const bool gemm_out = gemm && vx_gemm_fits_seg(H, vd, R, o, (size_t)vd, oseg);
+    if (vx_dn_prefill_packs(&pd)) {   // (a checkpointed window writes out_proj's operand itself)
+        if (vx_dn_prefill_window(ctx, &pd, p, op, tok_out)) return -1;
+        return vx_gemv_store(ctx, d->w_out, H, vd, op, R, tok_out, d->out, (size_t)H);
+    }
     if (vx_dn_prefill_into(ctx, &pd, p, gemm_out ? opk : nullptr)) return -1;
     if (gemm_out) return vx_gemm_store_packed(ctx, d->w_out, H, vd, opk, R, oseg, gws);
     if (vx_pack(ctx, o, (size_t)vd, R, vd, tok_out, op)) return -1;
