@@ -1,7 +1,8 @@
 """GPU tests of the token-tile projections (batches and prompts of more
-vectors than the operand groups of one pass hold) and of the checkpointed
-multi-step recurrence: both keep the sums of the single-vector, single-step
-calls, so every comparison is bit for bit.
+vectors than the operand groups of one pass hold), of the projections that
+read fp32 rows, and of the checkpointed multi-step recurrence: all keep the
+sums of the single-vector, single-step calls, so every comparison is bit for
+bit.
 
 Sizes: a small layer (hidden 160: fewer k-steps than the eight classes of the
 sum; 161 row blocks: no multiple of any workgroup's), batches at the edges of
@@ -39,13 +40,14 @@ def weights(ctx, r, conv_bf16=True):
     return dev
 
 
-def decode(ctx, dev, x, S, conv, skew=0):
-    """One layer step of x [B][HID]; the conv state `skew` floats off its buffer's start."""
+def decode(ctx, dev, x, S, conv, skew=0, xskew=0):
+    """One layer step of x [B][HID]; the conv state `skew` and x `xskew` floats off their buffers' starts."""
     from vx27_amd import lib as L
     B = x.shape[0]
     cs = np.concatenate([np.zeros(skew, np.float32), conv.ravel()])
-    Sd, cd, xb, ob = ctx.put(S), ctx.put(cs), ctx.put(x), ctx.buf(B * HID * 4)
-    d = L.DnLayerDesc(B, NQK, NV, 128, HID, xb.ptr, None, dev["w_in"].ptr, dev["w_out"].ptr, dev["conv_w"].ptr,
+    xs = np.concatenate([np.zeros(xskew, np.float32), x.ravel()])
+    Sd, cd, xb, ob = ctx.put(S), ctx.put(cs), ctx.put(xs), ctx.buf(B * HID * 4)
+    d = L.DnLayerDesc(B, NQK, NV, 128, HID, xb.ptr + 4 * xskew, None, dev["w_in"].ptr, dev["w_out"].ptr, dev["conv_w"].ptr,
                       dev["dt"], dev["A_log"].ptr, dev["dt_bias"].ptr, dev["norm_w"].ptr, Sd.ptr, cd.ptr + 4 * skew,
                       ob.ptr)
     L.check(L.lib().vx27_hip_dn_layer_decode(ctx.h, C.byref(d)), "dn_layer")
@@ -75,6 +77,17 @@ def test_decode_batch_bits(ctx, B, conv_bf16, skew):
         one = decode(ctx, dev, x[b:b + 1], S[b:b + 1], conv[b:b + 1])
         for g, o, n in zip(got, one, ("out", "S", "conv")):
             assert np.array_equal(g[b], o[0]), (n, b)
+
+
+@pytest.mark.parametrize("B", [1, 2, 5, 6])
+def test_rows_or_packed_bits(ctx, B):
+    """Up to 5 vectors are read as fp32 rows (16-byte aligned) or packed: the same bits."""
+    from vx27_amd import workloads as W
+    r = W.rng(34, f"rows_{B}")
+    dev = weights(ctx, r)
+    x, S, conv = inputs(r, B)
+    for a, b in zip(decode(ctx, dev, x, S, conv), decode(ctx, dev, x, S, conv, xskew=1)):
+        assert np.array_equal(a, b)
 
 
 @pytest.mark.parametrize("B,T", [(1, 1), (3, 2), (1, 8), (2, 9), (1, 17), (5, 7), (1, 36), (2, 33), (1, 70)])

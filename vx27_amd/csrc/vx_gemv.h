@@ -62,6 +62,11 @@ struct GemmOut {
 // in two halves.
 int vx_gemv_store_seg(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const uint16_t *packed, int B, bool tok,
                       const GemmOut &out, bool zeroed = false);
+// whether vx_gemv_store_x takes B vectors of K elements, x_stride apart
+bool vx_gemv_takes_x(int B, const float *x, size_t x_stride);
+// the same products and bits from the fp32 rows themselves, with no packed operand
+int vx_gemv_store_x(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const float *x, size_t x_stride, int B,
+                    const GemmOut &out);
 // the same to y[b*y_stride + n]
 int vx_gemv_store(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const uint16_t *packed, int B, bool tok,
                   float *y, size_t y_stride, bool zeroed = false);

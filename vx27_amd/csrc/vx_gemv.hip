@@ -94,6 +94,12 @@ __global__ __launch_bounds__(VX_WK_NW * 64) void gemv_wk_store(WkWeights wt, int
     vx_gemv_wk_body<RB, G>(wt, N, K, xp, Gt, g0, B, halves, epi);
 }
 
+template <int RB, int G>
+__global__ __launch_bounds__(VX_WK_NW * 64) void gemv_wk_store_x(WkWeights wt, int N, int K, WkRawX x, int B,
+                                                                WkStore epi) {
+    vx_gemv_wk_body<RB, G>(wt, N, K, x, G, 0, B, 1, epi);
+}
+
 // Epilogue of the token-tile form: the rows into their output segment
 // (fp32 or bf16; vec: 16-byte (bf16: 8-byte) aligned).
 struct TokStore {
@@ -200,6 +206,19 @@ int vx_gemv_store_seg(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const 
         VX_WK_DISPATCH(ctx, gemv_wk_store, p, (WkWeights{W, 0}), N, K, packed, Gt, g0, Bp, p.halves,
                        (WkStore{out, b0}));
     }
+    return 0;
+}
+
+bool vx_gemv_takes_x(int B, const float *x, size_t x_stride) {
+    return B <= WK_RAW_G * VX_PACK_GV && ((uintptr_t)x & 15) == 0 && x_stride % 4 == 0;
+}
+
+int vx_gemv_store_x(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const float *x, size_t x_stride, int B,
+                    const GemmOut &out) {
+    VX_REQUIRE(N > 0 && N % 16 == 0 && K > 0 && K % 32 == 0 && B >= 1 && vx_gemv_takes_x(B, x, x_stride),
+               "gemv: bad call on rows (N=%d K=%d B=%d)", N, K, B);
+    const WkPlan p = vx_gemv_wk_plan(N, K, ctx->n_cu, vx_pass_groups(B, 0));
+    VX_WK_RAW_DISPATCH(ctx, gemv_wk_store_x, p, (WkWeights{W, 0}), N, K, (WkRawX{x, x_stride}), B, (WkStore{out, 0}));
     return 0;
 }
 

@@ -22,6 +22,8 @@
 // measured slower on every projection shape of the model, with or without
 // device-scope fences.)
 #pragma once
+#include <type_traits>
+
 #include "vx_gemv.h"
 
 typedef __bf16 vx_bf16x8_t __attribute__((ext_vector_type(8)));
@@ -43,11 +45,12 @@ __host__ __device__ constexpr int vx_wk_max_rb(int G) {
     return G == 1 ? 20 : G == 2 ? 16 : G == 3 ? 10 : G == 4 ? 8 : G == 7 ? 4 : G == 10 ? 3 : 2;
 }
 // operand sets in a wave's ring: as many as fit beside the 4 RB G
-// accumulator registers in about 200 (an operand set takes 4 (RB + G)),
-// 1 .. VX_WK_DMAX
-__host__ __device__ constexpr int vx_wk_depth_raw(int RB, int G) { return (200 - 4 * RB * G) / (4 * (RB + G)); }
-__host__ __device__ constexpr int vx_wk_depth(int RB, int G) {
-    return vx_wk_depth_raw(RB, G) < 1 ? 1 : vx_wk_depth_raw(RB, G) > VX_WK_DMAX ? VX_WK_DMAX : vx_wk_depth_raw(RB, G);
+// accumulator registers in about 200 (an operand set takes 4 (RB + G); of
+// fp32 rows 4 (RB + 2 G), and the split about 40 registers more), 1 ..
+// VX_WK_DMAX
+__host__ __device__ constexpr int vx_wk_depth(int RB, int G, bool rows) {
+    const int d = (200 - 4 * RB * G - (rows ? 40 : 0)) / (4 * (RB + (rows ? 2 : 1) * G));
+    return d < 1 ? 1 : d > VX_WK_DMAX ? VX_WK_DMAX : d;
 }
 
 // k-steps per group of the tiled weight layout
@@ -99,14 +102,75 @@ struct WkRows {
 //       issues the loads the epilogue needs besides the sums (their latency
 //       then hides under the loop instead of trailing it)
 //   void operator()(int row0, int rows, const WkRows<RB, G> &, int tid, const Pre &) const
+// The operand of a pass, as a wave's ring holds it: tiles of the packed
+// operand, or (WkRaw, WK_RAW_G groups) the fp32 rows themselves, each lane
+// splitting its 8 elements of a k-step into the part that its operand column
+// holds.  Reading the rows spares the pack launch; the split is VALU work
+// beside the loads that bound the kernel, but every workgroup repeats it and
+// it grows with the groups: in_proj 27.6 us against 26.7 + 4.1 of the pack
+// with one group, 34.4 against 26.4 + 4.0 with two.
+struct WkPacked {
+    struct Tile { vx_bf16x8_t v; };
+    const vx_bf16x8_t *xb;
+    int Gt;
+    __device__ __forceinline__ WkPacked(const uint16_t *xp, int Gt, int g0, int, int lane)
+        : xb((const vx_bf16x8_t *)xp + (size_t)g0 * 64 + lane), Gt(Gt) {}
+    __device__ __forceinline__ Tile load(int s, int j, bool live, const vx_bf16x8_t *zt) const {
+        return Tile{*(live ? xb + ((size_t)s * Gt + j) * 64 : zt)};
+    }
+    __device__ __forceinline__ vx_bf16x8_t get(const Tile &t, int) const { return t.v; }
+};
+constexpr int WK_RAW_G = 1;
+struct WkRawX {           // fp32 rows, 16-byte aligned, a multiple of 4 floats apart
+    const float *x;
+    size_t stride;
+};
+struct WkRaw {
+    struct Tile { vx_floatx4_t a, b; };
+    const float *xr[WK_RAW_G];   // this lane's vector of each group, from k = 8 (lane / 16)
+    int part[WK_RAW_G];
+    __device__ __forceinline__ WkRaw(const WkRawX &x, int, int g0, int B, int lane) {
+#pragma unroll
+        for (int j = 0; j < WK_RAW_G; j++) {   // (column n: part n / Bj of vector n % Bj; the others feed unread columns)
+            const int Bj = min(VX_PACK_GV, max(B - VX_PACK_GV * j, 1)), n = min(lane & 15, 3 * Bj - 1);
+            part[j] = n / Bj;
+            xr[j] = x.x + (size_t)min(VX_PACK_GV * (g0 + j) + n % Bj, B - 1) * x.stride + 8 * (lane >> 4);
+        }
+    }
+    __device__ __forceinline__ Tile load(int s, int j, bool live, const vx_bf16x8_t *zt) const {
+        const vx_floatx4_t *p = live ? (const vx_floatx4_t *)(xr[j] + 32 * (size_t)s) : (const vx_floatx4_t *)zt;
+        return Tile{p[0], live ? p[1] : p[0]};
+    }
+    __device__ __forceinline__ vx_bf16x8_t get(const Tile &t, int j) const {
+        typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+        uint32_t u[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            float v[2] = {e < 2 ? t.a[2 * e] : t.b[2 * e - 4], e < 2 ? t.a[2 * e + 1] : t.b[2 * e - 3]};
+#pragma unroll
+            for (int p = 0; p < 3; p++) {   // part p = bf16 of what the earlier parts leave (exact in fp32)
+                const uint32_t h = __builtin_bit_cast(uint32_t, (bf16x2_t){(__bf16)v[0], (__bf16)v[1]});
+                u[e] = p == 0 || part[j] == p ? h : u[e];
+                v[0] = v[0] - __uint_as_float(h << 16);
+                v[1] = v[1] - __uint_as_float(h & 0xffff0000u);
+            }
+        }
+        vx_bf16x8_t r;
+        __builtin_memcpy(&r, u, 16);
+        return r;
+    }
+};
+
 // One pass covers the B vectors of groups g0 .. g0+G-1 of a packed operand
 // with Gt groups in all.  halves = 1: grid ceil(N / 16 RB), block 512;
 // halves = 2: grid 2 ceil(N / 16 RB), block 256, workgroup 2i + h running
 // waves 4h .. 4h+3 of row group i (the epilogue then gets only its half).
-template <int RB, int G, class Epi>
-__device__ __forceinline__ void vx_gemv_wk_body(const WkWeights &wt, int N, int K, const uint16_t *xp, int Gt,
-                                                int g0, int B, int halves, const Epi &epi) {
-    constexpr int NW = VX_WK_NW, D = vx_wk_depth(RB, G);
+// (The fp32 rows come as X = WkRawX, with g0 = 0: one pass.)
+template <int RB, int G, class Epi, class X>
+__device__ __forceinline__ void vx_gemv_wk_body(const WkWeights &wt, int N, int K, const X &xp, int Gt, int g0, int B,
+                                                int halves, const Epi &epi) {
+    typedef typename std::conditional<std::is_same<X, WkRawX>::value, WkRaw, WkPacked>::type Src;
+    constexpr int NW = VX_WK_NW, D = vx_wk_depth(RB, G, std::is_same<X, WkRawX>::value);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = halves == 2 ? (int)(blockIdx.x & 1) : 0;
@@ -127,31 +191,35 @@ __device__ __forceinline__ void vx_gemv_wk_body(const WkWeights &wt, int N, int 
 #pragma unroll
     for (int r = 0; r < RB; r++)   // dead blocks re-read block 0, never stored
         wp[r] = wt.base(rb0 + r < nb ? rb0 + r : 0, nb, K, kg, lane);
-    const vx_bf16x8_t *xb = (const vx_bf16x8_t *)xp + (size_t)g0 * 64 + lane;
+    const Src src(xp, Gt, g0, B, lane);
     // operands of k-step s; past the end (s >= k1) both operands come from
     // a zero tile, so that every path issues the same loads and MFMAs (the
     // waits before each MFMA then leave the later sets in flight) and the
     // extra products add exact zeros
     const vx_bf16x8_t *zt = vx_wk_zero + lane;
-    auto load = [&](int s, vx_bf16x8_t(&ao)[RB], vx_bf16x8_t(&bo)[G]) {
+    auto load = [&](int s, vx_bf16x8_t(&ao)[RB], typename Src::Tile(&bo)[G]) {
         const bool live = s < k1;
 #pragma unroll
-        for (int j = 0; j < G; j++) bo[j] = *(live ? xb + ((size_t)s * Gt + j) * 64 : zt);
+        for (int j = 0; j < G; j++) bo[j] = src.load(s, j, live, zt);
         const size_t off = wt.off(s, nb, kg);
 #pragma unroll
         for (int r = 0; r < RB; r++) ao[r] = *(live ? (const vx_bf16x8_t *)(wp[r] + off) : zt);
     };
-    auto mma = [&](const vx_bf16x8_t(&ao)[RB], const vx_bf16x8_t(&bo)[G]) {
+    auto mma = [&](const vx_bf16x8_t(&ao)[RB], const typename Src::Tile(&bo)[G]) {
+        vx_bf16x8_t o[G];
+#pragma unroll
+        for (int j = 0; j < G; j++) o[j] = src.get(bo[j], j);
 #pragma unroll
         for (int r = 0; r < RB; r++)
 #pragma unroll
             for (int j = 0; j < G; j++)
-                acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ao[r], bo[j], acc[r][j], 0, 0, 0);
+                acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ao[r], o[j], acc[r][j], 0, 0, 0);
     };
     // D operand sets in a ring: the loads of the next D - 1 k-steps of this
     // wave are in flight during the MFMAs of the current one (the branches
     // are uniform: s is a wave constant)
-    vx_bf16x8_t a[D][RB], b[D][G];
+    vx_bf16x8_t a[D][RB];
+    typename Src::Tile b[D][G];
 #pragma unroll
     for (int d = 0; d < D; d++) load(k0 + vw + d * NW, a[d], b[d]);
     for (int s = k0 + vw; s < k1; s += D * NW) {   // whole rounds of D k-steps
@@ -257,6 +325,7 @@ WkPlan vx_gemv_wk_plan(int N, int K, int n_cu, int G, bool allow_halves = false)
 #define VX_WK_ALL(X, ...)                                                                                        \
     VX_WK_RB_G1(X, __VA_ARGS__) VX_WK_RB_G2(X, __VA_ARGS__) VX_WK_RB_G3(X, __VA_ARGS__) VX_WK_RB_BIG(X, __VA_ARGS__)
 
+
 // Launch KERNEL<rb, g>(args...) for a plan (grid plan.grid, block 512 or
 // 256 for half workgroups).
 #define VX_WK_CASE(R, GG, ctx, KERNEL, p, ...)                                                                 \
@@ -268,6 +337,14 @@ WkPlan vx_gemv_wk_plan(int N, int K, int n_cu, int G, bool allow_halves = false)
     do {                                                                                      \
         switch (p.g * 64 + p.rb) {                                                            \
             VX_WK_ALL(VX_WK_CASE, ctx, KERNEL, p, __VA_ARGS__)                                \
+            default: VX_REQUIRE(false, "internal: no GEMV instance for rb=%d g=%d", p.rb, p.g); \
+        }                                                                                     \
+    } while (0)
+// the same for the kernels that read fp32 rows (G <= WK_RAW_G)
+#define VX_WK_RAW_DISPATCH(ctx, KERNEL, p, ...)                                               \
+    do {                                                                                      \
+        switch (p.g * 64 + p.rb) {                                                            \
+            VX_WK_RB_G1(VX_WK_CASE, ctx, KERNEL, p, __VA_ARGS__)                              \
             default: VX_REQUIRE(false, "internal: no GEMV instance for rb=%d g=%d", p.rb, p.g); \
         }                                                                                     \
     } while (0)

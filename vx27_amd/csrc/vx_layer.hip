@@ -263,6 +263,12 @@ __global__ __launch_bounds__(512) void gemv_dn_in_tok(TtArgs a, DnInTok epi) {
     vx_gemv_tok_body<RB>(a, epi);
 }
 
+template <int RB, int G>
+__global__ __launch_bounds__(VX_WK_NW * 64) void gemv_dn_in_x(WkWeights wt, int N, int K, WkRawX x, int B,
+                                                             DnInEpi epi) {
+    vx_gemv_wk_body<RB, G>(wt, N, K, x, G, 0, B, 1, epi);
+}
+
 __global__ void advance_pos_kernel(int *pos, int B) {
     const int b = threadIdx.x;
     if (b < B) pos[b] += 1;
@@ -350,7 +356,9 @@ extern "C" int vx27_hip_dn_layer_decode(vx27_hip_ctx *ctx, const vx27_dn_layer_d
     double2 *gates = (double2 *)p; p += gm_b;
     uint16_t *op = (uint16_t *)p;
 
-    if (!d->x_packed && vx_pack(ctx, d->x, (size_t)H, B, H, tok_in, xp)) return -1;
+    // (a few vectors are read as fp32 rows, with no pack launch)
+    const bool rows = !d->x_packed && vx_gemv_takes_x(B, d->x, (size_t)H);
+    if (!d->x_packed && !rows && vx_pack(ctx, d->x, (size_t)H, B, H, tok_in, xp)) return -1;
     if (tok_in) {
         const DnInArgs ea = {B, C, vd, nv, d->conv_state, d->conv_w, d->conv_w_dtype == VX27_BF16, act, z, ga, gb,
                              0, tok_out ? nullptr : d->out, (size_t)B * H};
@@ -366,7 +374,11 @@ extern "C" int vx27_hip_dn_layer_decode(vx27_hip_ctx *ctx, const vx27_dn_layer_d
         const DnInArgs ea = {Bp, C, vd, nv, d->conv_state, d->conv_w, d->conv_w_dtype == VX27_BF16, act, z, ga, gb,
                              b0, g0 == 0 ? d->out : nullptr, (size_t)B * H};
         const WkPlan wp = vx_gemv_wk_plan(Nin, H, ctx->n_cu, G);
-        VX_WK_DISPATCH(ctx, gemv_dn_in, wp, (WkWeights{d->w_in, 0}), Nin, H, xp, Gt, g0, Bp, (DnInEpi{ea}));
+        if (rows)
+            VX_WK_RAW_DISPATCH(ctx, gemv_dn_in_x, wp, (WkWeights{d->w_in, 0}), Nin, H, (WkRawX{d->x, (size_t)H}), Bp,
+                               (DnInEpi{ea}));
+        else
+            VX_WK_DISPATCH(ctx, gemv_dn_in, wp, (WkWeights{d->w_in, 0}), Nin, H, xp, Gt, g0, Bp, (DnInEpi{ea}));
     }
 
     DnArgs ra = {};
@@ -422,8 +434,12 @@ extern "C" int vx27_hip_gqa_layer_decode(vx27_hip_ctx *ctx, const vx27_gqa_layer
     uint16_t *ap = (uint16_t *)p; p += pk_a;
     void *gscr = p;
 
-    if (!d->x_packed && vx_pack(ctx, d->x, (size_t)H, B, H, tok_in, xp)) return -1;
-    if (vx_gemv_store(ctx, d->w_qkv, Nqkv, H, xp, B, tok_in, y, (size_t)Nqkv)) return -1;
+    if (!d->x_packed && vx_gemv_takes_x(B, d->x, (size_t)H)) {   // a few vectors: read as fp32 rows
+        if (vx_gemv_store_x(ctx, d->w_qkv, Nqkv, H, d->x, (size_t)H, B, vx_gemm_out1(y, (size_t)Nqkv))) return -1;
+    } else {
+        if (!d->x_packed && vx_pack(ctx, d->x, (size_t)H, B, H, tok_in, xp)) return -1;
+        if (vx_gemv_store(ctx, d->w_qkv, Nqkv, H, xp, B, tok_in, y, (size_t)Nqkv)) return -1;
+    }
     g.q = y; g.gate = y + hd; g.k_new = y + Nq; g.v_new = y + Nq + (size_t)d->n_kv * hd;
     g.out = nullptr;
     // the combine kernel clears out for o_proj's two halves
@@ -514,6 +530,8 @@ extern "C" int vx27_hip_dn_layer_prefill(vx27_hip_ctx *ctx, const vx27_dn_layer_
     seg.s[3] = GemmSeg{(C + vd + nv) / 16, 0, (size_t)nv, gb};
     if (gemm && nv % 16 == 0 && vx_gemm_fits_seg(Nin, H, R, d->x, (size_t)H, seg)) {
         if (vx_gemm_store_seg(ctx, d->w_in, Nin, H, d->x, (size_t)H, R, seg, gws)) return -1;
+    } else if (!gemm && nv % 16 == 0 && vx_gemv_takes_x(R, d->x, (size_t)H)) {
+        if (vx_gemv_store_x(ctx, d->w_in, Nin, H, d->x, (size_t)H, R, seg)) return -1;
     } else if (!gemm && nv % 16 == 0) {
         if (vx_pack(ctx, d->x, (size_t)H, R, H, tok_in, xp)) return -1;
         if (vx_gemv_store_seg(ctx, d->w_in, Nin, H, xp, R, tok_in, seg)) return -1;
@@ -596,6 +614,8 @@ extern "C" int vx27_hip_gqa_layer_prefill(vx27_hip_ctx *ctx, const vx27_gqa_laye
     seg.s[2] = GemmSeg{(Nq + kvd) / 16, 1, (size_t)kvd, vb};
     if (gemm && vx_gemm_fits_seg(Nqkv, H, R, d->x, (size_t)H, seg)) {
         if (vx_gemm_store_seg(ctx, d->w_qkv, Nqkv, H, d->x, (size_t)H, R, seg, gws)) return -1;
+    } else if (!gemm && vx_gemv_takes_x(R, d->x, (size_t)H)) {
+        if (vx_gemv_store_x(ctx, d->w_qkv, Nqkv, H, d->x, (size_t)H, R, seg)) return -1;
     } else if (!gemm) {
         if (vx_pack(ctx, d->x, (size_t)H, R, H, tok_in, xp)) return -1;
         if (vx_gemv_store_seg(ctx, d->w_qkv, Nqkv, H, xp, R, tok_in, seg)) return -1;
