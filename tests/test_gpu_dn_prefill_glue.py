@@ -221,3 +221,18 @@ def test_dn_prefill_checkpoints_and_commit(ctx):
         ctx.sync()
     Sn = Sd.download(g["S"].shape, np.float32)
     assert np.array_equal(Sn[0], g["S_ckpt"][0, 3]) and np.array_equal(Sn[1], g["S_ckpt"][1, 0])
+
+
+@pytest.mark.parametrize("flags", [ALL, 2 | 4 | 8])
+@pytest.mark.parametrize("nqk,nv,T,B,sub", [(2, 8, 130, 22, 6), (2, 10, 100, 26, 6), (16, 48, 70, 6, 2)])
+def test_dn_prefill_value_head_shares(ctx, nqk, nv, T, B, sub, flags):
+    """Few (chunk, value head)s: one preparation workgroup a value head; many:
+    one a QK head.  The same bits (4, 5 and 3 value heads a QK head)."""
+    from vx27_amd import workloads as W
+    d = W.dn_prefill_glue(B=B, T=T, nqk=nqk, nv=nv)
+    q = W.dn_prefill(B=B, T=T, nqk=nqk, nv=nv)
+    cut = {k: v[:sub] if k in ("x", "a", "b", "z", "S0", "conv0") else v for k, v in d.items()}
+    full = run_prefill(ctx, d, nqk, flags, bf16_qkv=[q[n] for n in "qkv"])
+    few = run_prefill(ctx, cut, nqk, flags, bf16_qkv=[q[n][:sub] for n in "qkv"])
+    for n in ("out", "S", "conv"):
+        assert np.array_equal(full[n][:sub], few[n]), n

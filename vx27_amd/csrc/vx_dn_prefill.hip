@@ -579,6 +579,7 @@ struct PrepTArgs {
     const void *conv_w;
     unsigned flags;
     const float *norm_w;
+    int parts;                      // workgroups a QK head: its value heads in `parts` shares (prept_parts)
 };
 
 // bf16 hi and lo of 8 floats
@@ -706,11 +707,12 @@ static_assert(2 * TN_TOTAL <= 160 * 1024, "two workgroups per CU");
 template <bool XIN>
 __global__ __launch_bounds__(256, 2) void dnp_prept(PrepTArgs p) {   // (two workgroups a CU: 256 registers)
     constexpr bool LO = true;   // (the glue's q, k, v always come with lo parts)
-    const int c = blockIdx.x, qh = blockIdx.y, b = blockIdx.z;
+    const int c = blockIdx.x, qh = blockIdx.y / p.parts, part = blockIdx.y % p.parts, b = blockIdx.z;
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, m = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool w2 = wave >= 2;
     const int nr = p.nv / p.nqk;
+    const int j0 = part * nr / p.parts, j1 = (part + 1) * nr / p.parts;   // its value heads of the QK head's nr
     const int t0 = c * CH;
     const int nvalid = min(CH, p.T - t0);
 
@@ -765,7 +767,7 @@ __global__ __launch_bounds__(256, 2) void dnp_prept(PrepTArgs p) {   // (two wor
             qlv[j] = (LO && ok) ? *(const uint4 *)(p.ql + off) : z4;
         }
     }
-    // the gates of value head jv < 4 by wave jv, while the rows arrive (lane =
+    // the gates of value head j0 + jv, jv < 4, by wave jv, while the rows arrive (lane =
     // token; masked tokens get beta = 0 and g = 0): beta, the cumulative
     // log-decay gam and e^gam, e^(gam_C - gam), written to LDS in its phase 3
     double g_gam = 0.0;
@@ -789,7 +791,7 @@ __global__ __launch_bounds__(256, 2) void dnp_prept(PrepTArgs p) {   // (two wor
         eg = (float)exp(sc);
         egc = (float)exp(sC - sc);
     };
-    if (wave < nr) gates(qh * nr + wave, g_gam, g_beta, g_eg, g_egc);
+    if (j0 + wave < j1) gates(qh * nr + j0 + wave, g_gam, g_beta, g_eg, g_egc);
     if (XIN) {
         // q and k from x as the glue's operations (vx27_qfwd.c:118-131): the
         // conv + SiLU, thread (tokens 16 wave .. +15, channels lane and
@@ -990,19 +992,20 @@ __global__ __launch_bounds__(256, 2) void dnp_prept(PrepTArgs p) {   // (two wor
     }
     // the K record: K^T operand tiles (rows = key dims in 8 blocks, k =
     // tokens in 2 steps) and the K and Q operand tiles (rows = tokens, k =
-    // one 32-dim block), four of each a wave
+    // one 32-dim block), four of each a wave (written by the first share)
     char *kr = p.krec + (((size_t)b * p.nqk + qh) * p.NC + c) * p.krec_bytes;
+    if (part == 0)
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int tile = wave * 4 + j, rb = tile >> 1, ks = tile & 1;
-        const int tr = tile >> 2, db = tile & 3;
-        const size_t o = ((size_t)tile * 64 + lane) * 16;
-        *(uint4 *)(kr + K_KT + o) = *(const uint4 *)&kT_h[(rb * 16 + m) * TP + 32 * ks + 8 * g];
-        *(uint4 *)(kr + K_KA + o) = *(const uint4 *)&k_rows[(tr * 16 + m) * RP + 32 * db + 8 * g];
-        *(uint4 *)(kr + K_QA + o) = *(const uint4 *)&q_rows[(tr * 16 + m) * RP + 32 * db + 8 * g];
-    }
+        for (int j = 0; j < 4; j++) {
+            const int tile = wave * 4 + j, rb = tile >> 1, ks = tile & 1;
+            const int tr = tile >> 2, db = tile & 3;
+            const size_t o = ((size_t)tile * 64 + lane) * 16;
+            *(uint4 *)(kr + K_KT + o) = *(const uint4 *)&kT_h[(rb * 16 + m) * TP + 32 * ks + 8 * g];
+            *(uint4 *)(kr + K_KA + o) = *(const uint4 *)&k_rows[(tr * 16 + m) * RP + 32 * db + 8 * g];
+            *(uint4 *)(kr + K_QA + o) = *(const uint4 *)&q_rows[(tr * 16 + m) * RP + 32 * db + 8 * g];
+        }
     __syncthreads();   // the rows and K^T hi are read out
-    if (LO) {          // the lo parts: k lo rows through R1 (K^T lo transposed into R0), then q lo rows
+    if (LO && part == 0) {   // the lo parts: k lo rows through R1 (K^T lo transposed into R0), then q lo rows
 #pragma unroll
         for (int j = 0; j < 4; j++) *(uint4 *)&k_rows[((tid >> 4) + 16 * j) * RP + 8 * seg] = kl[j];
         __syncthreads();
@@ -1046,8 +1049,8 @@ __global__ __launch_bounds__(256, 2) void dnp_prept(PrepTArgs p) {   // (two wor
             vx_dma16(base, (uint32_t)(((row - row0) * p.C + 4 * (lane & 15)) * 4), lds + 1024 * i);
         }
     };
-    for (int jv = 0; jv < nr; jv++) {
-        const int vh = qh * nr + jv;
+    for (int jv = 0; jv < j1 - j0; jv++) {
+        const int vh = qh * nr + j0 + jv;
         if (XIN) x_window(vh, 0, vx_lds_addr(smem + TN_R3));
         // ---- phase 3: the gates to LDS (computed in phase 1 by wave jv for
         // jv < 4, else here by wave 0)
@@ -2512,6 +2515,17 @@ size_t vx_dn_prefill_scratch(const vx27_dn_prefill_desc *d) {
     return al256(n_rec * (x3 ? XREC : REC)) + al256(n_rec * sizeof(float)) + glue_bytes;
 }
 
+// Shares of a QK head's value heads in the preparation: one workgroup a value
+// head while all of them fit one round of CUs at two a CU, else one a QK head
+// (which forms the q and k rows, the Gram products and the K record once for
+// its value heads).  A short prompt's few workgroups run alone on the chip, so
+// the launch lasts as long as one of them: at 187 tokens (48 workgroups of
+// three value heads, or 144 of one) 52.4 us in turn, 32.0 side by side.
+static int prept_parts(const vx27_dn_prefill_desc *d, int NC, int n_cu) {
+    const int nr = d->nv / d->nqk;
+    return (size_t)NC * d->nv * d->B <= (size_t)2 * n_cu ? nr : 1;
+}
+
 bool vx_dn_prefill_packs(const vx27_dn_prefill_desc *d) {
     DnArgs a = {};
     a.S = d->S;
@@ -2660,8 +2674,9 @@ int vx_dn_prefill_into(vx27_hip_ctx *ctx, const vx27_dn_prefill_desc *d, void *s
     if (trec) {
         char *rec = (char *)scr, *krec = (char *)scr + rec_bytes;
         PrepTArgs pa{d->T, d->nqk, d->nv, NC, q, k, ql, kl, v32, d->a, d->b, d->A_log, d->dt_bias, rec, krec,
-                     (int)krec_one, C, d->conv_w_dtype == VX27_BF16, d->x, d->conv_state, d->conv_w, d->flags, d->norm_w};
-        const dim3 pg((unsigned)NC, (unsigned)d->nqk, (unsigned)d->B);
+                     (int)krec_one, C, d->conv_w_dtype == VX27_BF16, d->x, d->conv_state, d->conv_w, d->flags, d->norm_w,
+                     prept_parts(d, NC, ctx->n_cu)};
+        const dim3 pg((unsigned)NC, (unsigned)(d->nqk * pa.parts), (unsigned)d->B);
         if (xin) VX_LAUNCH_NAMED(ctx, "dnp_prept", dnp_prept<true>, pg, dim3(256), pa);
         else VX_LAUNCH_NAMED(ctx, "dnp_prept", dnp_prept<false>, pg, dim3(256), pa);
         if (xin && conv_state_update()) return -1;   // prept read the state before token 0
