@@ -202,7 +202,7 @@ int vx_gemv_store_seg(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const 
     for (int g0 = 0; g0 < Gt; g0 += VX_PASS_G) {   // one pass up to 13 groups (65 vectors)
         const int b0 = g0 * VX_PACK_GV, G = vx_pass_groups(B, b0);
         const int Bp = std::min(B - b0, G * VX_PACK_GV);
-        const WkPlan p = vx_gemv_wk_plan(N, K, ctx->n_cu, G, zeroed);
+        const WkPlan p = vx_gemv_wk_plan(N, K, ctx->n_cu, G, zeroed && out.n == 1 && !out.s[0].bf16);
         VX_WK_DISPATCH(ctx, gemv_wk_store, p, (WkWeights{W, 0}), N, K, packed, Gt, g0, Bp, p.halves,
                        (WkStore{out, b0}));
     }

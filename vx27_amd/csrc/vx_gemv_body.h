@@ -269,16 +269,23 @@ struct WkStore {
     __device__ __forceinline__ Pre prefetch(int, int, int) const { return {}; }
     template <int RB, int G>
     __device__ __forceinline__ void operator()(int row0, int rows, const WkRows<RB, G> &c, int tid, const Pre &) const {
-        for (int t = tid; t < rows * c.B; t += c.nh * 4 * 64) {
+        if (out.n == 1 && !out.s[0].bf16) {
+            for (int t = tid; t < rows * c.B; t += c.nh * 4 * 64) {
+                const int r = t % rows, b = t / rows;
+                float *yp = (float *)out.s[0].p + (size_t)(b0 + b) * out.s[0].stride + row0 + r;
+                if (c.nh == 1) atomicAdd(yp, c.y(r, b));
+                else *yp = c.y(r, b);
+            }
+            return;
+        }
+        for (int t = tid; t < rows * c.B; t += c.nh * 4 * 64) {   // (whole workgroups)
             const int r = t % rows, b = t / rows, n = row0 + r;
             GemmSeg sg = out.s[0];
-            if (out.n > 1)
 #pragma unroll
-                for (int q = 1; q < VX_GEMM_SEGS; q++)
-                    if (q < out.n && n >= 16 * out.s[q].rb0) sg = out.s[q];
+            for (int q = 1; q < VX_GEMM_SEGS; q++)
+                if (q < out.n && n >= 16 * out.s[q].rb0) sg = out.s[q];
             const size_t o = (size_t)(b0 + b) * sg.stride + (n - 16 * sg.rb0);
             if (sg.bf16) ((uint16_t *)sg.p)[o] = vx_f32_to_bf16(c.y(r, b));
-            else if (c.nh == 1) atomicAdd((float *)sg.p + o, c.y(r, b));
             else ((float *)sg.p)[o] = c.y(r, b);
         }
     }
