@@ -40,18 +40,19 @@ def weights(ctx, r, conv_bf16=True):
     return dev
 
 
-def decode(ctx, dev, x, S, conv, skew=0, xskew=0):
-    """One layer step of x [B][HID]; the conv state `skew` and x `xskew` floats off their buffers' starts."""
+def decode(ctx, dev, x, S, conv, skew=0, xskew=0, in_place=False):
+    """One layer step of x [B][HID]; the conv state `skew` and x `xskew` floats off their buffers' starts; in_place: out is x."""
     from vx27_amd import lib as L
     B = x.shape[0]
     cs = np.concatenate([np.zeros(skew, np.float32), conv.ravel()])
     xs = np.concatenate([np.zeros(xskew, np.float32), x.ravel()])
     Sd, cd, xb, ob = ctx.put(S), ctx.put(cs), ctx.put(xs), ctx.buf(B * HID * 4)
+    op = xb if in_place else ob
     d = L.DnLayerDesc(B, NQK, NV, 128, HID, xb.ptr + 4 * xskew, None, dev["w_in"].ptr, dev["w_out"].ptr, dev["conv_w"].ptr,
                       dev["dt"], dev["A_log"].ptr, dev["dt_bias"].ptr, dev["norm_w"].ptr, Sd.ptr, cd.ptr + 4 * skew,
-                      ob.ptr)
+                      op.ptr)
     L.check(L.lib().vx27_hip_dn_layer_decode(ctx.h, C.byref(d)), "dn_layer")
-    res = (ob.download((B, HID), np.float32), Sd.download(S.shape, np.float32),
+    res = (op.download((B, HID), np.float32), Sd.download(S.shape, np.float32),
            cd.download(cs.shape, np.float32)[skew:].reshape(conv.shape))
     for b in (Sd, cd, xb, ob):
         b.free()
@@ -79,15 +80,17 @@ def test_decode_batch_bits(ctx, B, conv_bf16, skew):
             assert np.array_equal(g[b], o[0]), (n, b)
 
 
-@pytest.mark.parametrize("B", [1, 2, 5, 6])
+@pytest.mark.parametrize("B", [1, 2, 5, 6, 40])
 def test_rows_or_packed_bits(ctx, B):
-    """Up to 5 vectors are read as fp32 rows (16-byte aligned) or packed: the same bits."""
+    """Up to 5 vectors are read as fp32 rows, or packed (unaligned rows, rows
+    that the output overwrites): the same bits."""
     from vx27_amd import workloads as W
     r = W.rng(34, f"rows_{B}")
     dev = weights(ctx, r)
     x, S, conv = inputs(r, B)
-    for a, b in zip(decode(ctx, dev, x, S, conv), decode(ctx, dev, x, S, conv, xskew=1)):
-        assert np.array_equal(a, b)
+    for kw in ({"xskew": 1}, {"in_place": True}):
+        for a, b in zip(decode(ctx, dev, x, S, conv), decode(ctx, dev, x, S, conv, **kw)):
+            assert np.array_equal(a, b), kw
 
 
 @pytest.mark.parametrize("B,T", [(1, 1), (3, 2), (1, 8), (2, 9), (1, 17), (5, 7), (1, 36), (2, 33), (1, 70)])

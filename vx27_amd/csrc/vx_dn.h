@@ -98,6 +98,7 @@ struct DnArgs {
     float *conv_state;
     const void *conv_w;
     int conv_bf16;
+    int out_tiles;                // out_packed is in the token layout
     // activations: either x (fused conv) or q/k/v (already convolved or given)
     const float *x;
     const float *q, *k, *v;
@@ -111,7 +112,6 @@ struct DnArgs {
     float *out;                   // may be NULL when out_packed is set
     size_t out_tok;               // per-(t,b) stride of out
     uint16_t *out_packed;         // optional: out as the packed GEMV operand (steps == 1)
-    bool out_tiles;               // (in the token layout)
     // optional scratch [B][nv][128] for pre-norm outputs: lets a single-step
     // call with VX27_DN_OUT_GATE split each head's columns over workgroups
     // (the output norm then runs in a separate finish kernel)

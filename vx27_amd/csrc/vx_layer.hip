@@ -356,8 +356,11 @@ extern "C" int vx27_hip_dn_layer_decode(vx27_hip_ctx *ctx, const vx27_dn_layer_d
     double2 *gates = (double2 *)p; p += gm_b;
     uint16_t *op = (uint16_t *)p;
 
-    // (a few vectors are read as fp32 rows, with no pack launch)
-    const bool rows = !d->x_packed && vx_gemv_takes_x(B, d->x, (size_t)H);
+    // (a few vectors are read as fp32 rows, with no pack launch, unless out,
+    // which the projection's workgroups clear as they end, overlaps them)
+    const float *x0 = d->x, *x1 = x0 + (size_t)B * H, *o0 = d->out, *o1 = o0 + (size_t)B * H;
+    const bool rows = !d->x_packed && vx_gemv_takes_x(B, d->x, (size_t)H) &&
+                      ((uintptr_t)x1 <= (uintptr_t)o0 || (uintptr_t)o1 <= (uintptr_t)x0);
     if (!d->x_packed && !rows && vx_pack(ctx, d->x, (size_t)H, B, H, tok_in, xp)) return -1;
     if (tok_in) {
         const DnInArgs ea = {B, C, vd, nv, d->conv_state, d->conv_w, d->conv_w_dtype == VX27_BF16, act, z, ga, gb,
