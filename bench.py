@@ -551,19 +551,21 @@ def bench_layer_decode(ctx, B, Lctx=4096, iters=10):
         ctx.sync()
         wall = (time.perf_counter() - t0) / iters / len(lays)
         lib.vx27_hip_graph_destroy(g)
-        kernels = (("gemv_dn_in", "gemv_wk_store", "dn_step_kernel", "dn_step_split", "dn_decode_kernel")
-                   if kind == "dn" else ("gemv_wk_store", "gqa_prep", "gqa_split", "gqa_combine"))
+        store = ("gemv_wk_store", "gemv_wk_store_x", "gemv_tok_store")
+        dn_in = ("gemv_dn_in", "gemv_dn_in_x", "gemv_dn_in_tok")
+        kernels = (dn_in + store + ("dn_step_kernel", "dn_step_split", "dn_decode_kernel")
+                   if kind == "dn" else store + ("gqa_prep", "gqa_split", "gqa_combine"))
         _, per = _time_calls(ctx, call, kernels, iters)
         per = {k: v / len(lays) for k, v in per.items()}
         io = 2 * B * H * 4
         if kind == "dn":
             w_in, w_out = (C_ + vd + 2 * nv) * H * 2, H * vd * 2
             alg = w_in + w_out + 2 * B * nv * HD * HD * 4 + 2 * B * C_ * 3 * 4 + C_ * 4 * 2 + io
-            proj = {"gemv_dn_in": (w_in, per["gemv_dn_in"]), "gemv_wk_store": (w_out, per["gemv_wk_store"])}
+            proj = {"gemv_dn_in": (w_in, sum(per[k] for k in dn_in)), "gemv_wk_store": (w_out, sum(per[k] for k in store))}
         else:
             w_qkv, w_o = (24 * 2 * GQ + 2 * 4 * GQ) * H * 2, H * 24 * GQ * 2
             alg = w_qkv + w_o + B * 4 * (Lctx + 1) * GQ * 2 * 2 + B * 4 * GQ * 2 * 2 + io
-            proj = {"gemv_wk_store": (w_qkv + w_o, per["gemv_wk_store"])}
+            proj = {"gemv_wk_store": (w_qkv + w_o, sum(per[k] for k in store))}
         res[kind] = {
             "layers_timed": len(lays),
             "us_per_layer": round(wall * 1e6, 2), "us_per_token": round(wall / B * 1e6, 3),
