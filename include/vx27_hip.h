@@ -376,7 +376,7 @@ typedef struct {
 int vx27_hip_dn_layer_decode(vx27_hip_ctx *ctx, const vx27_dn_layer_desc *d);
 
 /* The mixer of one gated GQA layer for one decode token of B sequences
- * (any B; weights streamed once per 65 sequences)
+ * (any B; weights streamed once per 64 or 65 sequences)
  * (the attention branch of vx27_qlayer, vx27_qfwd.c:162-213):
  *   [q|gate interleaved per head | k | v] = W_qkv xn  (q_proj, k_proj, v_proj
  *                                      stacked: n_q*2*hd + 2*n_kv*hd rows),
@@ -402,9 +402,8 @@ int vx27_hip_gqa_layer_decode(vx27_hip_ctx *ctx, const vx27_gqa_layer_desc *d);
  * as vx27_engine_batch_step runs it per layer (vx27_run.c:187-238):
  * [qkv|z|a|b] = W_in x for every token, then vx27_hip_dn_prefill with every
  * glue stage (and the checkpoints, when given), then out = W_out o.  The
- * projections stream their weights once per 65 tokens, so this is for short
- * windows such as an MTP verify batch (the reference's batch is at most 8
- * tokens); a long prompt's projections belong in a GEMM.  x and out are
+ * projections read their weights once per 64 tokens below 256 tokens (and in
+ * the exact form), once per 256 in a GEMM from there.  x and out are
  * [B][T][hidden]; the other fields as vx27_dn_layer_desc; flags
  * VX27_DN_EXACT / VX27_DN_BF16 choose the prefill algorithm (checkpoints
  * imply the exact one, bit-identical to T vx27_hip_dn_layer_decode calls). */
