@@ -223,6 +223,22 @@ def test_gqa_edges_and_splits(ctx):
     assert np.abs(outs[-1][0] - want).max() < 1e-5
 
 
+@pytest.mark.parametrize("B,Lcap,want", [(20, 1664, 26), (23, 1472, 23), (171, 192, 3), (257, 192, 2)])
+def test_gqa_automatic_splits(ctx, B, Lcap, want):
+    """n_split = 0 takes ceil(2048 / (B n_kv)) splits (the sizes allow them all):
+    the bits of that count asked for, and not those of one split less."""
+    from vx27_amd import mixers as M, workloads as W
+    r = W.rng(26, f"splits_{B}")
+    lay = M.GatedGQALayer(ctx, B, Lcap, W.normal(r, 256, 0.1), W.normal(r, 256, 0.1))
+    for c in (lay.k_cache, lay.v_cache):   # the same rows for every sequence
+        c.upload(np.tile(W.bf16_bits(W.normal(r, 4 * Lcap * 256)), B))
+    pos = (Lcap - 1 - np.arange(B) % 90).astype(np.int32)
+    qg, k, v = W.normal(r, (B, 24, 512)), W.normal(r, (B, 4, 256)), W.normal(r, (B, 4, 256))
+    auto, asked, less = (lay.decode(pos, qg, k, v, n_split=n) for n in (0, want, want - 1))
+    assert np.array_equal(auto, asked)
+    assert not np.array_equal(auto, less)
+
+
 @pytest.mark.parametrize("rope_dim", [0, 32, 128, 256])
 def test_gqa_decode_rope_dims(ctx, rope_dim):
     """Other rotary widths (0: no rotation; 256: every dim rotated), ragged

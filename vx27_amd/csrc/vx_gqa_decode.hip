@@ -438,11 +438,10 @@ static int gqa_check(const vx27_gqa_desc *d) {
 static int gqa_n_split(const vx27_gqa_desc *d) {
     int n_split = d->n_split;
     if (n_split <= 0) {
-        // at most VX_SPLIT_WAVES waves over all (sequence, KV head) pairs (all
-        // resident at once: rounded up, a few waves ran a second round), at
-        // least VX_SPLIT_MINT tiles per wave
+        // ~VX_SPLIT_WAVES waves over all (sequence, KV head) pairs, at least
+        // VX_SPLIT_MINT tiles per wave
         const int tiles = d->L / TILE;
-        n_split = VX_SPLIT_WAVES / (d->B * d->n_kv);
+        n_split = (VX_SPLIT_WAVES + d->B * d->n_kv - 1) / (d->B * d->n_kv);
         if (n_split > (tiles + VX_SPLIT_MINT - 1) / VX_SPLIT_MINT) n_split = (tiles + VX_SPLIT_MINT - 1) / VX_SPLIT_MINT;
         if (n_split < 1) n_split = 1;
     }
