@@ -34,9 +34,10 @@ def ctx():
     c.close()
 
 
-def run_prefill(ctx, d, nqk, flags, ckpt=False, bf16_qkv=None):
+def run_prefill(ctx, d, nqk, flags, ckpt=False, bf16_qkv=None, skew=0):
     """vx27_hip_dn_prefill on workload d (dn_prefill_glue layout); returns
-    dict(out, S, conv[, S_ckpt, conv_ckpt])."""
+    dict(out, S, conv[, S_ckpt, conv_ckpt]).  ckpt "S": no conv checkpoint;
+    skew: the bytes that the checkpoints lie off their buffers' starts."""
     from vx27_amd import lib as L
     B, T, C_ = d["x"].shape
     nv = d["a"].shape[2]
@@ -60,16 +61,17 @@ def run_prefill(ctx, d, nqk, flags, ckpt=False, bf16_qkv=None):
     desc.norm_w, desc.z = put(d["norm_w"]), put(d["z"])
     sk = ck = None
     if ckpt:
-        sk = ctx.buf(B * T * nv * hd * hd * 4)
-        ck = ctx.buf(B * T * C_ * 3 * 4)
-        desc.S_ckpt, desc.conv_ckpt = sk.ptr, ck.ptr
+        sk = ctx.buf(B * T * nv * hd * hd * 4 + skew)
+        ck = ctx.buf(B * T * C_ * 3 * 4 + skew)
+        desc.S_ckpt, desc.conv_ckpt = sk.ptr + skew, None if ckpt == "S" else ck.ptr + skew
     L.check(L.lib().vx27_hip_dn_prefill(ctx.h, C.byref(desc)), "dn_prefill")
     ctx.sync()
     res = {"out": ob.download((B, T, nv, hd), np.float32), "S": Sd.download(d["S0"].shape, np.float32),
            "conv": cd.download(d["conv0"].shape, np.float32)}
     if ckpt:
-        res["S_ckpt"] = sk.download((B, T, nv, hd, hd), np.float32)
-        res["conv_ckpt"] = ck.download((B, T, C_, 3), np.float32)
+        at = lambda b, shape: b.download((b.nbytes // 4,), np.float32)[skew // 4:].reshape(shape)
+        res["S_ckpt"] = at(sk, (B, T, nv, hd, hd))
+        res["conv_ckpt"] = at(ck, (B, T, C_, 3))
         for bb in (sk, ck):
             bb.free()
     for bb in keep + [Sd, cd, ob]:
@@ -236,3 +238,42 @@ def test_dn_prefill_value_head_shares(ctx, nqk, nv, T, B, sub, flags):
     few = run_prefill(ctx, cut, nqk, flags, bf16_qkv=[q[n][:sub] for n in "qkv"])
     for n in ("out", "S", "conv"):
         assert np.array_equal(full[n][:sub], few[n]), n
+
+
+WINDOWS = [(1, 2, 8, 0), (1, 16, 48, 4), (10, 2, 10, 4), (2, 2, 50, 1 | 4), (17, 2, 8, 4), (2, 8, 8, 1 | 4),
+           (1, 16, 48, 4 | 8)]
+
+
+@pytest.mark.parametrize("skew", [0, 4])
+@pytest.mark.parametrize("B,nqk,nv,flags", WINDOWS)
+def test_dn_prefill_window_is_decode(ctx, B, nqk, nv, flags, skew):
+    """A checkpointed window runs the sums of vx27_hip_dn_decode called token
+    by token, whichever kernel that call takes: column-split heads (up to 128
+    ungated ones without the fused conv), one workgroup a head, the fused conv
+    (nv == nqk); checkpoints 16-byte aligned or not.  The states hold pairs of
+    rows of +-1e10 that cancel in every column sum (the keys and queries are
+    equal on the rows of a pair), so any other order of a sum changes bits."""
+    from vx27_amd import lib as L, mixers as M, workloads as W
+    T, hd = 4, 128
+    d = W.dn_prefill_glue(B=B, T=T, nqk=nqk, nv=nv, config=10)
+    d["S0"][:, :, :32] *= np.float32(5e11)
+    d["S0"][:, :, 96:] = -d["S0"][:, :, 31::-1]
+    C_ = d["x"].shape[2]
+    qk = 2 * nqk * hd
+    mirror = np.arange(C_)   # channels 96.. of a q or k head as its channels 31, 30, ..
+    mirror[:qk].reshape(-1, hd)[:, 96:] = mirror[:qk].reshape(-1, hd)[:, 31::-1]
+    d["x"] = np.ascontiguousarray(d["x"][:, :, mirror])
+    d["conv0"], d["conv_w_bf16"] = np.ascontiguousarray(d["conv0"][:, mirror]), d["conv_w_bf16"][mirror]
+    bq = [W.bf16_bits(a).reshape(B, T, -1, hd) for a in np.split(d["x"], [qk // 2, qk], axis=2)]
+    g = run_prefill(ctx, d, nqk, flags, ckpt=bool(flags & 1) or "S", bf16_qkv=bq, skew=skew)
+    lay = M.DeltaNetLayer(ctx, B, nqk, nv, d["A_log"], d["dt_bias"], norm_w=d["norm_w"], conv_w=d["conv_w_bf16"],
+                          conv_w_dtype=L.BF16, S0=d["S0"], conv0=d["conv0"])
+    for t in range(T):
+        at = lambda a: np.ascontiguousarray(a[:, t][None])
+        src = {"x": at(d["x"])} if flags & 1 else {n: at(W.bf16_to_f32(a)) for n, a in zip("qkv", bq)}
+        o = lay.decode(1, flags, at(d["a"]), at(d["b"]), z=at(d["z"]), **src)
+        assert np.array_equal(o[0], g["out"][:, t]), f"out token {t}"
+        assert np.array_equal(lay.state(), g["S_ckpt"][:, t]), f"S checkpoint {t}"
+        if flags & 1:
+            assert np.array_equal(lay.conv(), g["conv_ckpt"][:, t]), f"conv checkpoint {t}"
+    assert np.array_equal(lay.state(), g["S"])

@@ -83,6 +83,9 @@ __device__ __forceinline__ void block_sum2(double &u, double &v, double (*slot)[
 // Internal flag: q and k are final (normalised and scaled as step_exact
 // leaves them); the recurrence skips every q/k normalisation.
 constexpr unsigned VX_DN_QK_READY = 1u << 16;
+// Internal flag: no column split, as with the fused conv (for a call whose
+// decode form has it, run here on convolved inputs: the same sums).
+constexpr unsigned VX_DN_WHOLE_HEADS = 1u << 17;
 
 struct DnArgs {
     int B, nqk, nv, steps;
@@ -142,10 +145,14 @@ int vx_dn_gates(vx27_hip_ctx *ctx, size_t n, int nv, const float *ga, const floa
 
 // Launch the recurrence (one or more workgroups per (sequence, value head)).
 int vx_dn_recurrence(vx27_hip_ctx *ctx, const DnArgs &a);
+// Workgroups that share the columns of a head in a single-step call: 1, or
+// (few ungated heads) dn_step_split's, whose column sums run in another order.
+int vx_dn_step_cols(const DnArgs &a);
 // a.steps steps with the state after each written to S_ckpt
 // [B][steps][nv][128][128] too, bit-identical to single steps (q, k, v and the
-// raw gate inputs given, rows b steps + t; 16-byte aligned states:
-// vx_dn_steps_ok; out_packed: of all the rows).
+// raw gate inputs given, rows b steps + t; out_packed: of all the rows) where
+// those run a workgroup a head and the states are 16-byte aligned
+// (vx_dn_steps_ok).
 int vx_dn_steps(vx27_hip_ctx *ctx, const DnArgs &a, float *S_ckpt);
 bool vx_dn_steps_ok(const DnArgs &a, const float *S_ckpt);
 // Whether vx_dn_recurrence runs a call as one single-step kernel (which can

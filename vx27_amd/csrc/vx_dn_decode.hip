@@ -988,6 +988,12 @@ bool vx_dn_single_step(const DnArgs &a) {
     return VX_DN_STEP && a.steps == 1 && ((uintptr_t)a.S & 15) == 0;
 }
 
+int vx_dn_step_cols(const DnArgs &a) {
+    const int heads = a.B * a.nv;
+    if ((a.flags & (VX27_DN_OUT_GATE | VX_DN_WHOLE_HEADS)) || a.fused_conv || heads > 128) return 1;
+    return heads <= 32 ? 8 : heads <= 64 ? 4 : 2;
+}
+
 int vx_dn_recurrence(vx27_hip_ctx *ctx, const DnArgs &a_in) {
     DnArgs a = a_in;
     if (a.t_step == 0 && a.b_step == 0) {   // decode layout [steps][B]
@@ -1003,7 +1009,7 @@ int vx_dn_recurrence(vx27_hip_ctx *ctx, const DnArgs &a_in) {
     const bool gate = (a.flags & VX27_DN_OUT_GATE) != 0;
     if (vx_dn_single_step(a)) {
         // few heads, no fused conv and no output gate: columns split over CS workgroups
-        const int CS = (gate || a.fused_conv || heads > 128) ? 1 : heads <= 32 ? 8 : heads <= 64 ? 4 : 2;
+        const int CS = vx_dn_step_cols(a);
         if (CS > 1) {
             const dim3 grid((unsigned)(heads * CS));
             if (CS == 8) VX_LAUNCH_NAMED(ctx, "dn_step_split", dn_step_split<8>, grid, dim3(128), a);
@@ -1031,7 +1037,7 @@ int vx_dn_recurrence(vx27_hip_ctx *ctx, const DnArgs &a_in) {
     // kernel; splitting would need the dn_out_gate launch, which costs more
     // than the split gains.)
     int CS = 1;
-    if (!a.fused_conv && !gate)
+    if (!a.fused_conv && !gate && !(a.flags & VX_DN_WHOLE_HEADS))
         while (heads * CS < 512 && CS < 8) CS *= 2;
 #if defined(VX_DN_CS)
     if (CS > 1 || VX_DN_CS == 1) CS = VX_DN_CS;   // build-time override for tuning sweeps
@@ -1142,7 +1148,7 @@ int vx_dn_gates(vx27_hip_ctx *ctx, size_t n, int nv, const float *ga, const floa
 }
 
 bool vx_dn_steps_ok(const DnArgs &a, const float *S_ckpt) {
-    return (((uintptr_t)a.S | (uintptr_t)S_ckpt) & 15) == 0;
+    return (((uintptr_t)a.S | (uintptr_t)S_ckpt) & 15) == 0 && vx_dn_step_cols(a) == 1;
 }
 
 int vx_dn_steps(vx27_hip_ctx *ctx, const DnArgs &a, float *S_ckpt) {

@@ -2526,8 +2526,16 @@ static int prept_parts(const vx27_dn_prefill_desc *d, int NC, int n_cu) {
     return (size_t)NC * d->nv * d->B <= (size_t)2 * n_cu ? nr : 1;
 }
 
+// The flags under which the single steps of d run with the sums of the
+// decode call (which has the conv fused where nv == nqk).
+static unsigned dn_step_flags(const vx27_dn_prefill_desc *d) {
+    return (d->flags & (VX27_DN_PRE_RMS | VX27_DN_PRE_L2 | VX27_DN_OUT_GATE)) |
+           ((d->flags & VX27_DN_CONV) && d->nv == d->nqk ? VX_DN_WHOLE_HEADS : 0u);
+}
+
 bool vx_dn_prefill_packs(const vx27_dn_prefill_desc *d) {
     DnArgs a = {};
+    a.B = d->B; a.nv = d->nv; a.flags = dn_step_flags(d);
     a.S = d->S;
     return d->S_ckpt && vx_dn_steps_ok(a, d->S_ckpt);
 }
@@ -2575,7 +2583,9 @@ static int dn_prefill_exact(vx27_hip_ctx *ctx, const vx27_dn_prefill_desc *d, vo
         a.out = out_op ? nullptr : d->out; a.out_packed = out_op; a.out_tiles = tok;
         return vx_dn_steps(ctx, a, d->S_ckpt);
     }
-    // token by token, the state copied out after each (single-step kernel)
+    // token by token, the state copied out after each (single-step kernels:
+    // column-split heads, unaligned states)
+    a.flags = dn_step_flags(d);
     const size_t s_bytes = (size_t)d->nv * HD * HD * sizeof(float);
     for (int t = 0; t < d->T; t++) {
         DnArgs at = a;
