@@ -6,25 +6,14 @@
 // Packed activations: vectors go in groups of VX_PACK_GV, each group one
 // 16-column MFMA B operand (the three parts of its <= 5 vectors): layout
 // [K/32 k-steps][groups][64 lanes][8] bf16.
-// Above three groups the count is rounded up to 4, 7, 10 or 13 (one GEMV
-// pass covers up to 65 vectors; larger batches take whole multiples of 13):
-// the padding groups are never written and feed output columns nobody reads.
+// Above three groups the count is rounded up to 4, 7, 10 or 13 (65 vectors, one
+// pass over the weights): the padding groups are never written and feed output
+// columns nobody reads.
 constexpr int VX_PACK_GV = 5;
-constexpr int VX_PASS_G = 13;   // most groups per pass over the weights
-// groups of a pass holding the g <= VX_PASS_G groups that have vectors
-__host__ __device__ __forceinline__ int vx_round_groups(int g) {
-    return g <= 3 ? g : g <= 4 ? 4 : g <= 7 ? 7 : g <= 10 ? 10 : 13;
-}
-
+constexpr int VX_PASS_G = 13;   // most groups: 65 vectors
 __host__ __device__ __forceinline__ int vx_pack_groups(int B) {
     const int g = (B + VX_PACK_GV - 1) / VX_PACK_GV;
-    return g <= VX_PASS_G ? vx_round_groups(g) : (g + VX_PASS_G - 1) / VX_PASS_G * VX_PASS_G;
-}
-// groups of the pass that starts at vector b0 of B (its last group may be
-// followed by padding groups of the layout that the pass skips)
-__host__ __device__ __forceinline__ int vx_pass_groups(int B, int b0) {
-    const int g = (B - b0 + VX_PACK_GV - 1) / VX_PACK_GV;
-    return vx_round_groups(g < VX_PASS_G ? g : VX_PASS_G);
+    return g <= 3 ? g : g <= 4 ? 4 : g <= 7 ? 7 : g <= 10 ? 10 : 13;
 }
 // The token layout (tok) holds 16 vectors a tile, each part a tile of its own
 // (vx_gemv_tok.h): [K/32][ceil(B/16)][3 parts][64 lanes][8] bf16, lane (g, n)
@@ -55,8 +44,8 @@ struct GemmOut {
     GemmSeg s[VX_GEMM_SEGS];
 };
 // y_b[n] = sum over k of W[n][k] x_b[k] for tiled W and a packed x of B
-// vectors into output segments (operand groups: one pass over W for up to 65
-// vectors, passes of 13 groups beyond; tok: token tiles).  Each row's sum order
+// vectors into output segments (operand groups of up to 65 vectors: one pass
+// over W; tok: token tiles, one per 64 vectors).  Each row's sum order
 // is the same for any B and either layout.  zeroed: the output (fp32) holds
 // zeros, written by an earlier kernel on the stream, so the rows may be added
 // in two halves.

@@ -90,14 +90,14 @@ __global__ __launch_bounds__(64) void pack_w(const uint16_t *W, int K, uint16_t 
 
 template <int RB, int G>
 __global__ __launch_bounds__(VX_WK_NW * 64) void gemv_wk_store(WkWeights wt, int N, int K, const uint16_t *xp,
-                                                              int Gt, int g0, int B, int halves, WkStore epi) {
-    vx_gemv_wk_body<RB, G>(wt, N, K, xp, Gt, g0, B, halves, epi);
+                                                              int B, int halves, WkStore epi) {
+    vx_gemv_wk_body<RB, G>(wt, N, K, xp, B, halves, epi);
 }
 
 template <int RB, int G>
 __global__ __launch_bounds__(VX_WK_NW * 64) void gemv_wk_store_x(WkWeights wt, int N, int K, WkRawX x, int B,
                                                                 WkStore epi) {
-    vx_gemv_wk_body<RB, G>(wt, N, K, x, G, 0, B, 1, epi);
+    vx_gemv_wk_body<RB, G>(wt, N, K, x, B, 1, epi);
 }
 
 // Epilogue of the token-tile form: the rows into their output segment
@@ -198,14 +198,9 @@ int vx_gemv_store_seg(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const 
     VX_REQUIRE(N > 0 && N % 16 == 0 && K > 0 && K % 32 == 0 && B >= 1,
                "gemv: N must be a multiple of 16, K of 32, B >= 1 (N=%d K=%d B=%d)", N, K, B);
     if (tok) return gemv_tok(ctx, W, N, K, packed, B, out);
-    const int Gt = vx_pack_groups(B);
-    for (int g0 = 0; g0 < Gt; g0 += VX_PASS_G) {   // one pass up to 13 groups (65 vectors)
-        const int b0 = g0 * VX_PACK_GV, G = vx_pass_groups(B, b0);
-        const int Bp = std::min(B - b0, G * VX_PACK_GV);
-        const WkPlan p = vx_gemv_wk_plan(N, K, ctx->n_cu, G, zeroed && out.n == 1 && !out.s[0].bf16);
-        VX_WK_DISPATCH(ctx, gemv_wk_store, p, (WkWeights{W, 0}), N, K, packed, Gt, g0, Bp, p.halves,
-                       (WkStore{out, b0}));
-    }
+    VX_REQUIRE(B <= VX_PASS_G * VX_PACK_GV, "internal: %d vectors in operand groups", B);
+    const WkPlan p = vx_gemv_wk_plan(N, K, ctx->n_cu, vx_pack_groups(B), zeroed && out.n == 1 && !out.s[0].bf16);
+    VX_WK_DISPATCH(VX_WK_ALL, ctx, gemv_wk_store, p, (WkWeights{W, 0}), N, K, packed, B, p.halves, (WkStore{out, 0}));
     return 0;
 }
 
@@ -217,8 +212,9 @@ int vx_gemv_store_x(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, const fl
                     const GemmOut &out) {
     VX_REQUIRE(N > 0 && N % 16 == 0 && K > 0 && K % 32 == 0 && B >= 1 && vx_gemv_takes_x(B, x, x_stride),
                "gemv: bad call on rows (N=%d K=%d B=%d)", N, K, B);
-    const WkPlan p = vx_gemv_wk_plan(N, K, ctx->n_cu, vx_pass_groups(B, 0));
-    VX_WK_RAW_DISPATCH(ctx, gemv_wk_store_x, p, (WkWeights{W, 0}), N, K, (WkRawX{x, x_stride}), B, (WkStore{out, 0}));
+    const WkPlan p = vx_gemv_wk_plan(N, K, ctx->n_cu, vx_pack_groups(B));
+    VX_WK_DISPATCH(VX_WK_RB_G1, ctx, gemv_wk_store_x, p, (WkWeights{W, 0}), N, K, (WkRawX{x, x_stride}), B,
+                   (WkStore{out, 0}));
     return 0;
 }
 
@@ -264,10 +260,10 @@ extern "C" int vx27_hip_gemv_bf16(vx27_hip_ctx *ctx, const uint16_t *W, int N, i
     if (vx_ctx_scratch(ctx, vx_pack_bytes(K, Bp0, false), &scr)) return -1;
     uint16_t *packed = (uint16_t *)scr;
     for (int b0 = 0; b0 < B; b0 += VX_PASS_G * VX_PACK_GV) {
-        const int Bp = std::min(B - b0, VX_PASS_G * VX_PACK_GV), G = vx_pack_groups(Bp);
+        const int Bp = std::min(B - b0, VX_PASS_G * VX_PACK_GV);
         if (vx_pack(ctx, x + (size_t)b0 * x_stride, x_stride, Bp, K, false, packed)) return -1;
-        const WkPlan p = vx_gemv_wk_plan(N, K, ctx->n_cu, G);
-        VX_WK_DISPATCH(ctx, gemv_wk_store, p, (WkWeights{W, 1}), N, K, packed, G, 0, Bp, p.halves,
+        const WkPlan p = vx_gemv_wk_plan(N, K, ctx->n_cu, vx_pack_groups(Bp));
+        VX_WK_DISPATCH(VX_WK_ALL, ctx, gemv_wk_store, p, (WkWeights{W, 1}), N, K, packed, Bp, p.halves,
                        (WkStore{vx_gemm_out1(y, y_stride), b0}));
     }
     return 0;

@@ -79,7 +79,7 @@ struct WkWeights {
 };
 
 // Summed rows handed to an epilogue: y(r, b) for local row r < rows and
-// vector b < B of the pass (its groups g0 .. g0+G-1 of the packed operand):
+// vector b < B of the pass (groups 0 .. G-1 of the packed operand):
 // the nh halves' values added in order (nh = 1 in a half workgroup).
 template <int RB, int G>
 struct WkRows {
@@ -112,11 +112,11 @@ struct WkRows {
 struct WkPacked {
     struct Tile { vx_bf16x8_t v; };
     const vx_bf16x8_t *xb;
-    int Gt;
-    __device__ __forceinline__ WkPacked(const uint16_t *xp, int Gt, int g0, int, int lane)
-        : xb((const vx_bf16x8_t *)xp + (size_t)g0 * 64 + lane), Gt(Gt) {}
+    int G;
+    __device__ __forceinline__ WkPacked(const uint16_t *xp, int G, int, int lane)
+        : xb((const vx_bf16x8_t *)xp + lane), G(G) {}
     __device__ __forceinline__ Tile load(int s, int j, bool live, const vx_bf16x8_t *zt) const {
-        return Tile{*(live ? xb + ((size_t)s * Gt + j) * 64 : zt)};
+        return Tile{*(live ? xb + ((size_t)s * G + j) * 64 : zt)};
     }
     __device__ __forceinline__ vx_bf16x8_t get(const Tile &t, int) const { return t.v; }
 };
@@ -129,12 +129,12 @@ struct WkRaw {
     struct Tile { vx_floatx4_t a, b; };
     const float *xr[WK_RAW_G];   // this lane's vector of each group, from k = 8 (lane / 16)
     int part[WK_RAW_G];
-    __device__ __forceinline__ WkRaw(const WkRawX &x, int, int g0, int B, int lane) {
+    __device__ __forceinline__ WkRaw(const WkRawX &x, int, int B, int lane) {
 #pragma unroll
         for (int j = 0; j < WK_RAW_G; j++) {   // (column n: part n / Bj of vector n % Bj; the others feed unread columns)
             const int Bj = min(VX_PACK_GV, max(B - VX_PACK_GV * j, 1)), n = min(lane & 15, 3 * Bj - 1);
             part[j] = n / Bj;
-            xr[j] = x.x + (size_t)min(VX_PACK_GV * (g0 + j) + n % Bj, B - 1) * x.stride + 8 * (lane >> 4);
+            xr[j] = x.x + (size_t)min(VX_PACK_GV * j + n % Bj, B - 1) * x.stride + 8 * (lane >> 4);
         }
     }
     __device__ __forceinline__ Tile load(int s, int j, bool live, const vx_bf16x8_t *zt) const {
@@ -161,14 +161,13 @@ struct WkRaw {
     }
 };
 
-// One pass covers the B vectors of groups g0 .. g0+G-1 of a packed operand
-// with Gt groups in all.  halves = 1: grid ceil(N / 16 RB), block 512;
+// One pass covers the B vectors of a packed operand of G groups.  halves = 1: grid ceil(N / 16 RB), block 512;
 // halves = 2: grid 2 ceil(N / 16 RB), block 256, workgroup 2i + h running
 // waves 4h .. 4h+3 of row group i (the epilogue then gets only its half).
-// (The fp32 rows come as X = WkRawX, with g0 = 0: one pass.)
+// (The fp32 rows come as X = WkRawX.)
 template <int RB, int G, class Epi, class X>
-__device__ __forceinline__ void vx_gemv_wk_body(const WkWeights &wt, int N, int K, const X &xp, int Gt, int g0, int B,
-                                                int halves, const Epi &epi) {
+__device__ __forceinline__ void vx_gemv_wk_body(const WkWeights &wt, int N, int K, const X &xp, int B, int halves,
+                                                const Epi &epi) {
     typedef typename std::conditional<std::is_same<X, WkRawX>::value, WkRaw, WkPacked>::type Src;
     constexpr int NW = VX_WK_NW, D = vx_wk_depth(RB, G, std::is_same<X, WkRawX>::value);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -191,7 +190,7 @@ __device__ __forceinline__ void vx_gemv_wk_body(const WkWeights &wt, int N, int 
 #pragma unroll
     for (int r = 0; r < RB; r++)   // dead blocks re-read block 0, never stored
         wp[r] = wt.base(rb0 + r < nb ? rb0 + r : 0, nb, K, kg, lane);
-    const Src src(xp, Gt, g0, B, lane);
+    const Src src(xp, G, B, lane);
     // operands of k-step s; past the end (s >= k1) both operands come from
     // a zero tile, so that every path issues the same loads and MFMAs (the
     // waits before each MFMA then leave the later sets in flight) and the
@@ -324,34 +323,28 @@ WkPlan vx_gemv_wk_plan(int N, int K, int n_cu, int G, bool allow_halves = false)
 #define VX_WK_RB_G3(X, ...)                                                                                      \
     X(1, 3, __VA_ARGS__) X(2, 3, __VA_ARGS__) X(3, 3, __VA_ARGS__) X(4, 3, __VA_ARGS__) X(5, 3, __VA_ARGS__)    \
     X(6, 3, __VA_ARGS__) X(7, 3, __VA_ARGS__) X(8, 3, __VA_ARGS__) X(9, 3, __VA_ARGS__) X(10, 3, __VA_ARGS__)
-#define VX_WK_RB_BIG(X, ...)                                                                                     \
+#define VX_WK_RB_G47(X, ...)                                                                                     \
     X(1, 4, __VA_ARGS__) X(2, 4, __VA_ARGS__) X(3, 4, __VA_ARGS__) X(4, 4, __VA_ARGS__) X(5, 4, __VA_ARGS__)    \
     X(6, 4, __VA_ARGS__) X(7, 4, __VA_ARGS__) X(8, 4, __VA_ARGS__) X(1, 7, __VA_ARGS__) X(2, 7, __VA_ARGS__)    \
-    X(3, 7, __VA_ARGS__) X(4, 7, __VA_ARGS__) X(1, 10, __VA_ARGS__) X(2, 10, __VA_ARGS__) X(3, 10, __VA_ARGS__) \
-    X(1, 13, __VA_ARGS__) X(2, 13, __VA_ARGS__)
-#define VX_WK_ALL(X, ...)                                                                                        \
-    VX_WK_RB_G1(X, __VA_ARGS__) VX_WK_RB_G2(X, __VA_ARGS__) VX_WK_RB_G3(X, __VA_ARGS__) VX_WK_RB_BIG(X, __VA_ARGS__)
-
+    X(3, 7, __VA_ARGS__) X(4, 7, __VA_ARGS__)
+#define VX_WK_RB_BIG(X, ...)                                                                                     \
+    X(1, 10, __VA_ARGS__) X(2, 10, __VA_ARGS__) X(3, 10, __VA_ARGS__) X(1, 13, __VA_ARGS__) X(2, 13, __VA_ARGS__)
+// (up to 7 groups: all that an input projection hands over as operand groups)
+#define VX_WK_G7(X, ...)                                                                                         \
+    VX_WK_RB_G1(X, __VA_ARGS__) VX_WK_RB_G2(X, __VA_ARGS__) VX_WK_RB_G3(X, __VA_ARGS__) VX_WK_RB_G47(X, __VA_ARGS__)
+#define VX_WK_ALL(X, ...) VX_WK_G7(X, __VA_ARGS__) VX_WK_RB_BIG(X, __VA_ARGS__)
 
 // Launch KERNEL<rb, g>(args...) for a plan (grid plan.grid, block 512 or
-// 256 for half workgroups).
+// 256 for half workgroups), of the instances LIST.
 #define VX_WK_CASE(R, GG, ctx, KERNEL, p, ...)                                                                 \
     case GG * 64 + R:                                                                                          \
         VX_LAUNCH_NAMED(ctx, #KERNEL, (KERNEL<R, GG>), dim3((unsigned)p.grid),                                 \
                         dim3(VX_WK_NW * 64 / p.halves), __VA_ARGS__);                                          \
         break;
-#define VX_WK_DISPATCH(ctx, KERNEL, p, ...)                                                   \
+#define VX_WK_DISPATCH(LIST, ctx, KERNEL, p, ...)                                             \
     do {                                                                                      \
         switch (p.g * 64 + p.rb) {                                                            \
-            VX_WK_ALL(VX_WK_CASE, ctx, KERNEL, p, __VA_ARGS__)                                \
-            default: VX_REQUIRE(false, "internal: no GEMV instance for rb=%d g=%d", p.rb, p.g); \
-        }                                                                                     \
-    } while (0)
-// the same for the kernels that read fp32 rows (G <= WK_RAW_G)
-#define VX_WK_RAW_DISPATCH(ctx, KERNEL, p, ...)                                               \
-    do {                                                                                      \
-        switch (p.g * 64 + p.rb) {                                                            \
-            VX_WK_RB_G1(VX_WK_CASE, ctx, KERNEL, p, __VA_ARGS__)                              \
+            LIST(VX_WK_CASE, ctx, KERNEL, p, __VA_ARGS__)                                     \
             default: VX_REQUIRE(false, "internal: no GEMV instance for rb=%d g=%d", p.rb, p.g); \
         }                                                                                     \
     } while (0)

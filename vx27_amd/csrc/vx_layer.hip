@@ -37,7 +37,6 @@ struct DnInArgs {
     int conv_bf16;
     float *act, *z;
     float *ga, *gb;   // the a and b rows, [B][nv] each (the step kernel maps them to the gates)
-    int b0;   // first vector of this pass (the pass's B vectors are b0 .. b0+B-1)
     float *zero;    // optional: zero_n floats cleared (the output out_proj adds its halves into)
     size_t zero_n;
 };
@@ -79,7 +78,7 @@ struct DnInEpi {
 #pragma unroll
             for (int b = 0; b < DN_PREB; b++)
                 if (b < a.B) {
-                    const float *sp = a.conv_state + ((size_t)(a.b0 + b) * a.C + n) * 3;
+                    const float *sp = a.conv_state + ((size_t)b * a.C + n) * 3;
                     p.st[b][0] = sp[0];
                     p.st[b][1] = sp[1];
                     p.st[b][2] = sp[2];
@@ -116,16 +115,16 @@ struct DnInEpi {
             }
             float w[4];
             taps(u, w);
-            float *sp = a.conv_state + ((size_t)(a.b0 + b) * a.C + n) * 3;
+            float *sp = a.conv_state + ((size_t)b * a.C + n) * 3;
             float st[3] = {sp[0], sp[1], sp[2]};
-            a.act[(size_t)(a.b0 + b) * a.C + n] = conv_step(st, w, y);
+            a.act[(size_t)b * a.C + n] = conv_step(st, w, y);
             sp[0] = st[0]; sp[1] = st[1]; sp[2] = st[2];
         } else if (n < a.C + a.vd) {
-            a.z[(size_t)(a.b0 + b) * a.vd + (n - a.C)] = y;
+            a.z[(size_t)b * a.vd + (n - a.C)] = y;
         } else if (n < a.C + a.vd + a.nv) {
-            a.ga[(size_t)(a.b0 + b) * a.nv + (n - a.C - a.vd)] = y;
+            a.ga[(size_t)b * a.nv + (n - a.C - a.vd)] = y;
         } else {
-            a.gb[(size_t)(a.b0 + b) * a.nv + (n - a.C - a.vd - a.nv)] = y;
+            a.gb[(size_t)b * a.nv + (n - a.C - a.vd - a.nv)] = y;
         }
     }
     template <int RB, int G>
@@ -149,8 +148,8 @@ struct DnInEpi {
             float w[4];
             taps(p.w, w);
             auto step = [&](int b, float st[3]) {
-                float *sp = a.conv_state + ((size_t)(a.b0 + b) * a.C + n) * 3;
-                a.act[(size_t)(a.b0 + b) * a.C + n] = conv_step(st, w, c.y(tid, b));
+                float *sp = a.conv_state + ((size_t)b * a.C + n) * 3;
+                a.act[(size_t)b * a.C + n] = conv_step(st, w, c.y(tid, b));
                 sp[0] = st[0]; sp[1] = st[1]; sp[2] = st[2];
             };
 #pragma unroll
@@ -160,21 +159,21 @@ struct DnInEpi {
                     step(b, st);
                 }
         } else if (n < a.C + a.vd) {         // z
-            for (int b = 0; b < a.B; b++) a.z[(size_t)(a.b0 + b) * a.vd + (n - a.C)] = c.y(tid, b);
+            for (int b = 0; b < a.B; b++) a.z[(size_t)b * a.vd + (n - a.C)] = c.y(tid, b);
         } else if (n < a.C + a.vd + a.nv) {  // a
             const int vh = n - a.C - a.vd;
-            for (int b = 0; b < a.B; b++) a.ga[(size_t)(a.b0 + b) * a.nv + vh] = c.y(tid, b);
+            for (int b = 0; b < a.B; b++) a.ga[(size_t)b * a.nv + vh] = c.y(tid, b);
         } else {                             // b
             const int vh = n - a.C - a.vd - a.nv;
-            for (int b = 0; b < a.B; b++) a.gb[(size_t)(a.b0 + b) * a.nv + vh] = c.y(tid, b);
+            for (int b = 0; b < a.B; b++) a.gb[(size_t)b * a.nv + vh] = c.y(tid, b);
         }
     }
 };
 
 template <int RB, int G>
-__global__ __launch_bounds__(VX_WK_NW * 64) void gemv_dn_in(WkWeights wt, int N, int K, const uint16_t *xp, int Gt,
-                                                           int g0, int B, DnInEpi epi) {
-    vx_gemv_wk_body<RB, G>(wt, N, K, xp, Gt, g0, B, 1, epi);   // whole rows (the conv needs them)
+__global__ __launch_bounds__(VX_WK_NW * 64) void gemv_dn_in(WkWeights wt, int N, int K, const uint16_t *xp, int B,
+                                                           DnInEpi epi) {
+    vx_gemv_wk_body<RB, G>(wt, N, K, xp, B, 1, epi);   // whole rows (the conv needs them)
 }
 
 // The same epilogue after the token-tile form (vx_gemv_tok.h), four rows of
@@ -266,7 +265,7 @@ __global__ __launch_bounds__(512) void gemv_dn_in_tok(TtArgs a, DnInTok epi) {
 template <int RB, int G>
 __global__ __launch_bounds__(VX_WK_NW * 64) void gemv_dn_in_x(WkWeights wt, int N, int K, WkRawX x, int B,
                                                              DnInEpi epi) {
-    vx_gemv_wk_body<RB, G>(wt, N, K, x, G, 0, B, 1, epi);
+    vx_gemv_wk_body<RB, G>(wt, N, K, x, B, 1, epi);
 }
 
 __global__ void advance_pos_kernel(int *pos, int B) {
@@ -362,26 +361,20 @@ extern "C" int vx27_hip_dn_layer_decode(vx27_hip_ctx *ctx, const vx27_dn_layer_d
     const bool rows = !d->x_packed && vx_gemv_takes_x(B, d->x, (size_t)H) &&
                       ((uintptr_t)x1 <= (uintptr_t)o0 || (uintptr_t)o1 <= (uintptr_t)x0);
     if (!d->x_packed && !rows && vx_pack(ctx, d->x, (size_t)H, B, H, tok_in, xp)) return -1;
+    // the projection clears out, so that out_proj may add its two halves into
+    // it (the same bits as whole rows; its token tiles store whole rows)
+    const DnInArgs ea = {B, C, vd, nv, d->conv_state, d->conv_w, d->conv_w_dtype == VX27_BF16, act, z, ga, gb,
+                         tok_out ? nullptr : d->out, (size_t)B * H};
     if (tok_in) {
-        const DnInArgs ea = {B, C, vd, nv, d->conv_state, d->conv_w, d->conv_w_dtype == VX27_BF16, act, z, ga, gb,
-                             0, tok_out ? nullptr : d->out, (size_t)B * H};
         const TtPlan p = vx_gemv_tok_plan(d->w_in, xp, Nin, H, B, ctx->n_cu);
         VX_TT_DISPATCH(ctx, gemv_dn_in_tok, p, (DnInTok{ea, ((uintptr_t)d->conv_state & 15) == 0}));
-    }
-    const int Gt = tok_in ? 0 : vx_pack_groups(B);
-    for (int g0 = 0; g0 < Gt; g0 += VX_PASS_G) {   // one pass over W_in up to 13 groups (65 vectors)
-        const int b0 = g0 * VX_PACK_GV, G = vx_pass_groups(B, b0);
-        const int Bp = B - b0 < G * VX_PACK_GV ? B - b0 : G * VX_PACK_GV;
-        // the first pass clears out, so that out_proj may add its two halves
-        // into it (the same bits as whole rows)
-        const DnInArgs ea = {Bp, C, vd, nv, d->conv_state, d->conv_w, d->conv_w_dtype == VX27_BF16, act, z, ga, gb,
-                             b0, g0 == 0 ? d->out : nullptr, (size_t)B * H};
-        const WkPlan wp = vx_gemv_wk_plan(Nin, H, ctx->n_cu, G);
+    } else {
+        const WkPlan wp = vx_gemv_wk_plan(Nin, H, ctx->n_cu, vx_pack_groups(B));
         if (rows)
-            VX_WK_RAW_DISPATCH(ctx, gemv_dn_in_x, wp, (WkWeights{d->w_in, 0}), Nin, H, (WkRawX{d->x, (size_t)H}), Bp,
-                               (DnInEpi{ea}));
+            VX_WK_DISPATCH(VX_WK_RB_G1, ctx, gemv_dn_in_x, wp, (WkWeights{d->w_in, 0}), Nin, H,
+                           (WkRawX{d->x, (size_t)H}), B, (DnInEpi{ea}));
         else
-            VX_WK_DISPATCH(ctx, gemv_dn_in, wp, (WkWeights{d->w_in, 0}), Nin, H, xp, Gt, g0, Bp, (DnInEpi{ea}));
+            VX_WK_DISPATCH(VX_WK_G7, ctx, gemv_dn_in, wp, (WkWeights{d->w_in, 0}), Nin, H, xp, B, (DnInEpi{ea}));
     }
 
     DnArgs ra = {};
