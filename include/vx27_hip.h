@@ -171,7 +171,7 @@ int vx27_hip_dn_decode(vx27_hip_ctx *ctx, const vx27_dn_desc *d);
  *   exact (VX27_DN_EXACT, or whenever a checkpoint is asked for): the
  *     decode kernels' fp32 recurrence token by token, the reference's own
  *     arithmetic (bit-identical to vx27_hip_dn_decode called token by
- *     token when checkpoints are written).  Meant for short windows such as
+ *     token when state checkpoints are written).  Meant for short windows such as
  *     an MTP verify batch (the reference's batch is at most 8 tokens).
  * Inputs are [B][T][...] (token t of sequence b at row b*T + t). */
 #define VX27_DN_EXACT 16u
@@ -351,8 +351,8 @@ int vx27_hip_gemm_bf16(vx27_hip_ctx *ctx, const uint16_t *W_tiled, int N, int K,
 int vx27_hip_pack_weights_bf16(vx27_hip_ctx *ctx, const uint16_t *W, int N, int K, uint16_t *W_tiled);
 
 /* The mixer of one Gated DeltaNet layer for one decode token of B
- * sequences (any B; the projections stream their weights once per 65
- * sequences), from the layer input xn to the out_proj output (the DeltaNet
+ * sequences (any B; the weights are streamed once per 64 sequences, the
+ * output projection's once for 65 too), from the layer input xn to the out_proj output (the DeltaNet
  * branch of vx27_qlayer, vx27_qfwd.c:102-153):
  *   [qkv | z | a | b] = W_in xn      (in_proj_qkv, in_proj_z, in_proj_a, in_proj_b
  *                                      stacked row-wise: C + nv*hd + 2*nv rows)
@@ -376,7 +376,7 @@ typedef struct {
 int vx27_hip_dn_layer_decode(vx27_hip_ctx *ctx, const vx27_dn_layer_desc *d);
 
 /* The mixer of one gated GQA layer for one decode token of B sequences
- * (any B; weights streamed once per 64 or 65 sequences)
+ * (any B; weights streamed as in vx27_hip_dn_layer_decode)
  * (the attention branch of vx27_qlayer, vx27_qfwd.c:162-213):
  *   [q|gate interleaved per head | k | v] = W_qkv xn  (q_proj, k_proj, v_proj
  *                                      stacked: n_q*2*hd + 2*n_kv*hd rows),
@@ -402,11 +402,11 @@ int vx27_hip_gqa_layer_decode(vx27_hip_ctx *ctx, const vx27_gqa_layer_desc *d);
  * as vx27_engine_batch_step runs it per layer (vx27_run.c:187-238):
  * [qkv|z|a|b] = W_in x for every token, then vx27_hip_dn_prefill with every
  * glue stage (and the checkpoints, when given), then out = W_out o.  The
- * projections read their weights once per 64 tokens below 256 tokens (and in
- * the exact form), once per 256 in a GEMM from there.  x and out are
+ * projections read their weights as in vx27_hip_dn_layer_decode (for tokens)
+ * below 256 tokens and in the exact form, once per 256 tokens in a GEMM from there.  x and out are
  * [B][T][hidden]; the other fields as vx27_dn_layer_desc; flags
  * VX27_DN_EXACT / VX27_DN_BF16 choose the prefill algorithm (checkpoints
- * imply the exact one, bit-identical to T vx27_hip_dn_layer_decode calls). */
+ * imply the exact one; with S_ckpt bit-identical to T vx27_hip_dn_layer_decode calls). */
 typedef struct {
     int B, T, nqk, nv, hd, hidden;
     unsigned flags;

@@ -114,7 +114,7 @@ struct DnArgs {
     size_t z_tok;                 // per-(t,b) stride of z
     float *out;                   // may be NULL when out_packed is set
     size_t out_tok;               // per-(t,b) stride of out
-    uint16_t *out_packed;         // optional: out as the packed GEMV operand (steps == 1)
+    uint16_t *out_packed;         // optional: out as the packed GEMV operand (of one step, or of vx_dn_steps's window)
     // optional scratch [B][nv][128] for pre-norm outputs: lets a single-step
     // call with VX27_DN_OUT_GATE split each head's columns over workgroups
     // (the output norm then runs in a separate finish kernel)

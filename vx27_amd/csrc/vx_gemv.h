@@ -18,12 +18,21 @@ __host__ __device__ __forceinline__ int vx_pack_groups(int B) {
 // The token layout (tok) holds 16 vectors a tile, each part a tile of its own
 // (vx_gemv_tok.h): [K/32][ceil(B/16)][3 parts][64 lanes][8] bf16, lane (g, n)
 // of block j: vector 16 j + n, k 8g .. 8g+7.
-// The wide input projections take it from 36 vectors (8 operand groups, padded
-// to 10: their whole-K workgroups no longer fit one round of CUs: in_proj at 64
-// vectors 93 against 70 us, GQA qkv at 40 49 against 42); the narrow output
-// projections, whose whole-K grid fits one round at any group count (36 us
-// against 40 at 64 vectors), where the groups would need a second pass over
-// the weights.
+// The wide input projections take it from 36 vectors, where the operand groups
+// are padded from 8 to 10 and the GQA qkv's whole-K workgroups (2 row blocks)
+// no longer fit one round of CUs (in_proj's run two rounds from 5 groups on and
+// three with 13).  The narrow output projections, whose whole-K grid fits one round at any
+// group count, take it where the groups would need a second pass over the
+// weights.  Kernel trace, us, weights streamed from HBM, groups / token tiles:
+//   vectors       36        40        64         65         66         129
+//   in_proj    95 / 64   97 / 65  127 / 75  127 / 124  153 / 124  220 / 172
+//   GQA qkv    65 / 47   66 / 46   82 / 50   82 / 84   104 / 83   144 / 111
+//   out_proj                                            59 / 45    83 / 48
+// (65 pads to two 64-vector tiles and only breaks even there; the layer calls at
+// 65 still gain, 252 -> 243 us and 164 -> 157.)  With 7 groups, 21 to 35
+// vectors, in_proj takes 65 to 69 us and qkv 42; token tiles were not timed
+// there.  out_proj at 64 vectors, one layer's weights in the last-level cache:
+// 36 us against 40 in token tiles.
 constexpr int VX_TOK_IN = 36, VX_TOK_OUT = VX_PASS_G * VX_PACK_GV + 1;
 __host__ __device__ __forceinline__ bool vx_tok_in(int B) { return B >= VX_TOK_IN; }
 __host__ __device__ __forceinline__ bool vx_tok_out(int B) { return B >= VX_TOK_OUT; }

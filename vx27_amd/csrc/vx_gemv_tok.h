@@ -1,5 +1,5 @@
 // Token-tile form of the skinny projections, for more vectors than a few
-// MFMA operand groups hold (VX_TOK_MIN and up): the same exact three-part
+// MFMA operand groups hold (VX_TOK_IN, VX_TOK_OUT: vx_gemv.h): the same exact three-part
 // products and the same bits as the whole-K GEMV (vx_gemv_body.h), shared
 // with the kernels that put their own epilogue after it (vx_layer.hip).
 //
@@ -24,10 +24,14 @@
 // y0 in LDS.
 //
 // Measured (kernel trace): in_proj 16480 x 5120 of 64 vectors 70 us against
-// 93 as whole-K workgroups (515 of them, of 2 row blocks: three rounds), of 187
+// 93 as whole-K workgroups (515 of them, of 2 row blocks: three rounds) with one
+// layer's weights in the last-level cache, 75 against 127 from HBM; of 187
 // vectors 153 us against 284 in three passes, out_proj 5120 x 6144 of 187
-// vectors 53 us against 117; a step takes about 0.36 + 0.055 RB us, 0.042 RB
-// of it MFMA.  The operand as fp32 tiles split in registers (a third less L2
+// vectors 53 us against 117.  A step takes about 0.36 + 0.055 RB us over the
+// three rounds of 187 vectors, 0.042 RB of it MFMA; one round of 64 vectors
+// takes 20 us more than its 80 steps would, unaccounted for.  Timing-only
+// copies of the 187-token layer (252 us): without the loads 209, without the
+// MFMAs 235, without the LDS reads 245.  The operand as fp32 tiles split in registers (a third less L2
 // traffic) was slower, 85 us at 64 vectors: the split's VALU work adds to a
 // step.  Separate, deeper rings for the weights changed nothing.
 #pragma once

@@ -3,8 +3,9 @@
 //
 // DeltaNet layer (vx27_qfwd.c:102-153), one decode token of B sequences:
 //   gemv_dn_in               [qkv | z | a | b] projection with its epilogue
-//                            (DnInEpi): causal conv/SiLU on qkv (state in
-//                            place), z, a and b copied out
+//                            (DnInEpi; DnInTok after the token tiles): causal
+//                            conv/SiLU on qkv (state in place), z, a and b
+//                            copied out
 //   dn_step_kernel           gates (decay from a, beta from b), q/k
 //                            normalisation chain, exact step, gated output
 //                            norm, output written as the packed operand of
@@ -15,8 +16,13 @@
 //   gqa_prep / gqa_split / gqa_combine (vx_gqa_decode.hip; the combine
 //                            writes the packed operand of W_o)
 //   gemv_wk_store(W_o)       -> out
-// (the GEMVs are whole-K workgroups with the reduction in LDS:
-// vx_gemv_body.h)
+// (the GEMVs are whole-K workgroups with the reduction in LDS, on fp32 rows or
+// operand groups: vx_gemv_body.h; or token tiles: vx_gemv_tok.h; the rule is in
+// vx_gemv.h)
+// The layer over T tokens: the same projections, or the GEMM (vx_gemm.hip) from
+// 256 rows on, around the chunked or the exact prefill (vx_dn_prefill.hip); a
+// window with state checkpoints writes W_out's packed operand itself
+// (dn_steps_kernel).
 #include <math.h>
 
 #include <algorithm>
@@ -496,9 +502,9 @@ extern "C" int vx27_hip_dn_layer_prefill(vx27_hip_ctx *ctx, const vx27_dn_layer_
     const size_t inner = vx_dn_prefill_scratch(&pd);
     // [qkv | z | a | b] = W_in x for all B*T tokens: a long prompt of the
     // chunked form in the GEMM (W_in read once per 256 tokens, x as two bf16
-    // parts, as precise as the chunked products); otherwise one pass over W_in
-    // per 65 tokens with each row summed in the same order as in a decode step
-    // (the exact form is bit-identical to T decode calls)
+    // parts, as precise as the chunked products); otherwise the GEMV forms, with
+    // each row summed in the same order as in a decode step (with state
+    // checkpoints the call is bit-identical to T decode calls)
     const bool exact = (d->flags & VX27_DN_EXACT) || d->S_ckpt || d->conv_ckpt;
     const bool gemm = !exact && R >= VX_GEMM_MIN_ROWS;
     // (the long-prompt GEMMs' workspace, one region for both)
